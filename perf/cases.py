@@ -80,13 +80,13 @@ def draw(rng):
     if kind == "ffn":
         packed = rng.random() < 0.4
         return {"kind": kind, "type": "q6_k" if packed else rng.choice(["q6_k", "q5_k", "q4_k"]), "packed": packed,
-                "n_embd": rng.choice([2048, 4096, 4096]), "n_ff": 2048 * rng.randint(2, 6),
+                "n_embd": rng.choice([2048, 4096, 4096]), "n_ff": 2048 * rng.randint(2, 6) if packed else 256 * rng.randint(16, 48),
                 "ncols": rng.choice([1, 2, rng.randint(3, 15), 16])}
     if kind == "head":
         return {"kind": kind, "n_embd": rng.choice([2048, 4096]), "n_vocab": _log(rng, 5000, VOCAB), "ncols": rng.choice([1, 2])}
     if kind == "gdn":
-        h_k, h_v = rng.choice([(16, 32), (16, 32), (8, 16), (4, 8)])
-        return {"kind": kind, "h_k": h_k, "h_v": h_v, "ntok": rng.choice([1, 2, rng.randint(3, 15), 16])}
+        h_k = rng.choice([16, rng.randint(2, 15), rng.randint(2, 15)])
+        return {"kind": kind, "h_k": h_k, "h_v": 2 * h_k, "ntok": rng.choice([1, 2, rng.randint(3, 15), rng.randint(3, 16)])}
     if kind == "attn":
         n_head, n_kv = rng.choice([(16, 4), (16, 4), (8, 2)])
         ntok = rng.choice([1, 2, rng.randint(3, 15), 16])
