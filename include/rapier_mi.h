@@ -116,6 +116,11 @@ int rmi_native_q6_k_mmvq_packed(const void* w_packed, const void* x_q8_1, float*
                                 void* stream);
 int rmi_native_q6_k_mmvq_packed_res_n(const void* w_packed, const void* x_q8_1, float* y, const float* res,
                                       float* partials, int n_in, int n_out, int ncols, void* stream);
+/* The packed GEMV for whole prompts: 1..4096 columns in one weight pass on the matrix cores, each column bitwise the
+ * GEMV's (res and partials NULL: plain).  ws: rmi_q6_k_gemm_workspace_bytes of scratch; y, res and ws 16-byte aligned. */
+size_t rmi_q6_k_gemm_workspace_bytes(int n_in, int ncols);
+int rmi_q6_k_gemm_packed(const void* w_packed, const void* x_q8_1, float* y, const float* res, float* partials,
+                         int n_in, int n_out, int ncols, void* ws, void* stream);
 
 /* Q8_0 x Q8_1.  Replaces native_q8_0_mmvq (mmvq:3732-3736; dot mmvq:835-847) and native_q8_0_mmvq_res
  * (mmvq:3326-3339, kernel mmvq:3142-3185). */

@@ -48,6 +48,8 @@ SIGNATURES = {
     "rmi_rms_quant_apply_self": (_i, [_vp, _vp, _vp, _i, _f, _i, _vp]),
     "rmi_native_q6_k_mmvq_packed": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "rmi_native_q6_k_mmvq_packed_res_n": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
+    "rmi_q6_k_gemm_workspace_bytes": (_sz, [_i, _i]),
+    "rmi_q6_k_gemm_packed": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp]),
     "rmi_q6_k_block_dots": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "rmi_native_q6_k_mmvq_packed_norm": (_i, [_vp, _vp, _vp, _vp, _f, _vp, _i, _i, _i, _vp]),
     "rmi_native_q6_k_swiglu_packed_norm": (_i, [_vp, _vp, _vp, _vp, _f, _vp, _i, _i, _i, _vp]),
@@ -268,6 +270,19 @@ def native_q6_k_mmvq_packed_res_n(w_packed, x_q8_1, y, res, partials, n_in: int,
                                   stream=None):
     _call("rmi_native_q6_k_mmvq_packed_res_n", _p(w_packed), _p(x_q8_1), _p(y), _p(res), _p(partials), n_in, n_out,
           ncols, _stream(stream))
+
+
+def q6_k_gemm_workspace_bytes(n_in: int, ncols: int) -> int:
+    n = lib().rmi_q6_k_gemm_workspace_bytes(n_in, ncols)
+    if n == 0:
+        raise ValueError(last_error())
+    return n
+
+
+def q6_k_gemm_packed(w_packed, x_q8_1, y, res, partials, n_in: int, n_out: int, ncols: int, ws, stream=None):
+    """the packed GEMV over 1..4096 columns in one weight pass; each column bitwise the GEMV's"""
+    _call("rmi_q6_k_gemm_packed", _p(w_packed), _p(x_q8_1), _p(y), _p(res), _p(partials), n_in, n_out, ncols, _p(ws),
+          _stream(stream))
 
 
 def q6_k_block_dots(w, x_q8_1, out, n_in: int, n_out: int, stream=None):

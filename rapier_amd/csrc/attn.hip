@@ -16,8 +16,10 @@
 // Query t sees positions <= pos[0] + t.  Chunk boundaries depend only on the query's position, so a verify column's
 // result is bitwise the single-token result at the same position.
 #include "rmi_common.h"
+#include "ingest.h"
 #include "rope.h"
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -638,21 +640,27 @@ __global__ __launch_bounds__(HD) void gqa_merge_kernel(const float* __restrict__
 
 using namespace rmi;
 
-extern "C" int rmi_attn_prep_rope(const float* q3, int q3_stride, const float* qn, const float* kn,
-                                  uint16_t* kcache, uint16_t* vcache, const int* pos, float* qout, int n_head,
-                                  int n_kv, int head_dim, int n_rot, const rmi_rope_params* rope, float eps, int ntok,
-                                  int max_ctx, void* stream) {
+int rmi::attn_prep_cols(const float* q3, int q3_stride, const float* qn, const float* kn, uint16_t* kcache,
+                        uint16_t* vcache, const int* pos, float* qout, int n_head, int n_kv, int head_dim, int n_rot,
+                        const rmi_rope_params* rope, float eps, int ntok, int limit, int max_ctx, hipStream_t stream) {
     if (head_dim != HD || n_head <= 0 || n_kv <= 0 || n_head % n_kv || n_rot < 0 || n_rot > HD || n_rot % 2 ||
-        ntok < 1 || ntok > kMaxCols || !rope || !(rope->freq_base > 1.0f))
+        ntok < 1 || ntok > limit || !rope || !(rope->freq_base > 1.0f))
         return fail(RMI_ERR_SHAPE, "attn_prep: invalid arguments");
     if (!aligned4(q3) || !aligned4(qn) || !aligned4(kn) || !kcache || !vcache || !aligned4(pos) || !aligned4(qout))
         return fail(RMI_ERR_POINTER, "attn_prep: invalid arguments");
     Yarn y{};
     if (!yarn_setup(*rope, n_rot, &y)) return fail(RMI_ERR_SHAPE, "attn_prep: invalid YaRN parameters");
-    hipLaunchKernelGGL(attn_prep_kernel, dim3(ntok, n_head + 2 * n_kv), dim3(HD), 0, static_cast<hipStream_t>(stream),
-                       q3, q3_stride, qn, kn, kcache, vcache, pos, qout, n_head, n_kv, n_rot, max_ctx, rope->freq_base,
+    hipLaunchKernelGGL(attn_prep_kernel, dim3(ntok, n_head + 2 * n_kv), dim3(HD), 0, stream, q3, q3_stride, qn, kn, kcache, vcache, pos, qout, n_head, n_kv, n_rot, max_ctx, rope->freq_base,
                        eps, y);
     return launch_status("attn_prep");
+}
+
+extern "C" int rmi_attn_prep_rope(const float* q3, int q3_stride, const float* qn, const float* kn,
+                                  uint16_t* kcache, uint16_t* vcache, const int* pos, float* qout, int n_head,
+                                  int n_kv, int head_dim, int n_rot, const rmi_rope_params* rope, float eps, int ntok,
+                                  int max_ctx, void* stream) {
+    return attn_prep_cols(q3, q3_stride, qn, kn, kcache, vcache, pos, qout, n_head, n_kv, head_dim, n_rot, rope, eps,
+                          ntok, kMaxCols, max_ctx, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rmi_attn_prep(const float* q3, int q3_stride, const float* qn, const float* kn, uint16_t* kcache,
@@ -736,6 +744,35 @@ int scratch_address(hipStream_t stream, float** out) {
 
 }  // namespace
 }  // namespace rmi
+
+// Tokens pos[0] .. pos[0] + ntok - 1 of a wide ingest chunk: launches of up to `per` tokens, the grid cut at the chunks
+// that the last position (known to the host) reaches.  A slot's arithmetic does not depend on its launch or group.
+int rmi::flash_wide(const float* q, const uint16_t* kcache, const uint16_t* vcache, const int* pos, int pos0,
+                    const float* gate_src, int gate_stride, uint8_t* q8, int q8_stride, void* workspace, int per,
+                    int n_head, int n_kv, int head_dim, int ntok, int max_ctx, int nsub, float scale, hipStream_t s) {
+    int nchunks = 0;
+    RMI_TRY(flash_decode_check(q, kcache, vcache, pos, gate_src, nullptr, q8, n_head, n_kv, head_dim, 1, max_ctx, nsub,
+                               &nchunks));
+    const int G = n_head / n_kv, chunk_len = SUB * nsub;
+    if (per < 1 || per * G > 65535 || ntok < 1 || pos0 < 0 || pos0 + ntok > max_ctx || !aligned16(workspace))
+        return fail(RMI_ERR_SHAPE, "flash_wide: invalid arguments");
+    const int slots = (per * G + SLOTS - 1) / SLOTS * SLOTS;
+    for (int t = 0; t < ntok; t += per) {
+        const int nt = std::min(per, ntok - t);
+        RMI_TRY(flash_decode(q + static_cast<size_t>(t) * n_head * HD, kcache, vcache, pos + t,
+                             gate_src + static_cast<size_t>(t) * gate_stride, gate_stride, nullptr, 0,
+                             q8 + static_cast<size_t>(t) * q8_stride, q8_stride, static_cast<float*>(workspace), slots,
+                             n_head, n_kv, nt, std::min(nchunks, (pos0 + t + nt - 1) / chunk_len + 1), nsub, max_ctx,
+                             scale, s));
+    }
+    return RMI_OK;
+}
+
+size_t rmi::flash_wide_bytes(int max_ctx, int n_head, int n_kv, int nsub, int per) {
+    const size_t chunks = (static_cast<size_t>(max_ctx) + SUB * nsub - 1) / (SUB * nsub);
+    const size_t slots = (static_cast<size_t>(per) * (n_head / n_kv) + SLOTS - 1) / SLOTS * SLOTS;
+    return chunks * n_kv * slots * REC * sizeof(float);
+}
 
 extern "C" int rmi_gqa_flash_decode(const float* q, const uint16_t* kcache, const uint16_t* vcache, const int* pos,
                                     const float* gate_src, int gate_stride, float* y, int y_stride, uint8_t* q8,

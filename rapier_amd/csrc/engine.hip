@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "../../include/rapier_mi_engine.h"
+#include "ingest.h"
 
 namespace rmi {
 namespace {
@@ -36,6 +37,11 @@ namespace {
 constexpr int kS = 128;          // GDN state size
 constexpr int kRingCap = 1 << 16;
 constexpr int kChunk = kMaxCols;  // ingest chunk: prompt tokens per weight pass
+// Wide ingest chunks: up to kWideCols tokens per pass over the weights, while at least kWideMin are left (below that
+// the GEMM's 128-column tile costs more than the 16-column passes).  1999 tokens of the 9B model: 456 -> 141 ms.
+constexpr int kWideCols = 1024;
+constexpr int kWideMin = 64;
+constexpr int kWideAttnTok = 128;   // tokens per attention launch of a wide chunk (its split-K records: 64 MiB at 2K)
 constexpr int kAttnSlots = 64;    // query vectors per KV head one rmi_gqa_flash_decode launch takes
 
 int hip_check(hipError_t e, const char* what) {
@@ -130,13 +136,17 @@ struct Engine {
     int qkvz_rows = 0, q3_rows = 0, gdn_v = 0, attn_q = 0, max_in = 0;
 
     int* ints = nullptr;            // kNumSlots
-    int* cints = nullptr;           // ingest chunk: trunk tokens [0, 16), positions [16, 32)
+    int cols = kChunk;              // columns of the activation buffers: kChunk, or a wide chunk's
+    bool wide = false;              // prompts run in wide chunks (every matrix packed)
+    int wide_pos = 0;               // position of the wide chunk's first token
+    void *gemm_ws = nullptr, *gdn_ws = nullptr;   // wide chunks: the GEMM operand, the GDN scratch
+    int* cints = nullptr;           // ingest chunk: trunk tokens [0, cols), positions [cols, 2 cols)
     int* prompt = nullptr;          // ingest: the prompt's token ids, indexed by position
     int* ring = nullptr;            // emitted tokens
     int* ref_tok = nullptr;         // forced-acceptance reference stream, indexed by position
     uint8_t* pattern = nullptr;     // forced-acceptance pattern, indexed by round
 
-    // activations (kChunk columns; decode uses the first two).  hsave / hpart hold kChunk + 1 columns: an ingest chunk
+    // activations (cols columns; decode uses the first two).  hsave / hpart hold cols + 1 columns: an ingest chunk
     // writes its hidden to columns 1..nc, so that column c - 1 is the draft input of column c
     float *x = nullptr, *part = nullptr, *proj = nullptr, *ug = nullptr, *y = nullptr, *logits = nullptr;
     float *hsave = nullptr, *hpart = nullptr, *hzero = nullptr, *pzero = nullptr, *qbuf = nullptr;
@@ -340,12 +350,12 @@ __global__ __launch_bounds__(256) void first_tail_kernel(int* st, const uint64_t
 }
 
 // ingest chunk set-up: nc prompt tokens from position st[kPos]; column c is token prompt[pos + c] at pos + c
-__global__ void chunk_setup_kernel(const int* st, const int* prompt, int* cints, int nc) {
-    const int c = threadIdx.x;
+__global__ void chunk_setup_kernel(const int* st, const int* prompt, int* cints, int cols, int nc) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
     const int p = st[kPos] + c;
     if (c < nc) {
         cints[c] = prompt[p];
-        cints[kChunk + c] = p;
+        cints[cols + c] = p;
     }
 }
 
@@ -405,6 +415,7 @@ int make_mat(Engine& e, Mat& m, int n_out, int n_in, uint64_t seed, bool swiglu 
 }
 
 int gemv(Engine& e, const Mat& m, const uint8_t* xq, float* y, int nc) {
+    if (nc > kChunk) return q6k_packed_gemm(m.w, xq, y, nullptr, nullptr, m.n_in, m.n_out, nc, e.gemm_ws, e.s);
     if (!m.parts.empty()) {   // mixed-type group: each part, each column, into its rows (qw:1296-1308)
         const size_t xcol = q81_bytes(m.n_in);
         for (int c = 0; c < nc; ++c) {
@@ -421,6 +432,7 @@ int gemv(Engine& e, const Mat& m, const uint8_t* xq, float* y, int nc) {
 }
 
 int gemv_res(Engine& e, const Mat& m, const uint8_t* xq, float* x, float* part, int nc) {
+    if (nc > kChunk) return q6k_packed_gemm(m.w, xq, x, x, part, m.n_in, m.n_out, nc, e.gemm_ws, e.s);
     if (m.packed) return rmi_native_q6_k_mmvq_packed_res_n(m.w, xq, x, x, part, m.n_in, m.n_out, nc, e.s);
     switch (m.type) {
         case 14: return rmi_native_q6_k_mmvq_res_n(m.w, xq, x, x, part, m.n_in, m.n_out, nc, e.s);
@@ -524,9 +536,9 @@ int norm_input(Engine& e, const float* x, const float* part, const float* w, int
     *xq = e.q8a;
     if (e.norm_self) {
         e.norm_self = false;
-        return rmi_rms_quant_apply_self(x + xs, w, e.q8a, c.n_embd, c.eps, nc, e.s);
+        return rms_quant_self_cols(x + xs, w, e.q8a, c.n_embd, c.eps, nc, e.cols, e.s);
     }
-    return rmi_rms_quant_apply(x + xs, w, part + ps, e.q8a, c.n_embd, c.eps, nc, e.s);
+    return rms_quant_cols(x + xs, w, part + ps, e.q8a, c.n_embd, c.eps, nc, e.cols, e.s);
 }
 
 // A norm and the GEMV behind it in one launch (rms_quant_apply quantized into the GEMV's own stage, the same bits):
@@ -559,9 +571,9 @@ int ffn(Engine& e, Layer& L, float* x, float* part, int nc) {
     } else {
         RMI_TRY(gemv(e, L.upgate, xq, e.ug, nc));
         if (L.upgate.swiglu_ff)
-            RMI_TRY(rmi_swiglu_quant_interleaved(e.ug, e.q8f, c.n_ff, nc, 2 * c.n_ff, e.s));
+            RMI_TRY(swiglu_interleaved_cols(e.ug, e.q8f, c.n_ff, nc, 2 * c.n_ff, e.cols, e.s));
         else
-            RMI_TRY(rmi_swiglu_quant(e.ug, e.ug + c.n_ff, e.q8f, c.n_ff, nc, 2 * c.n_ff, e.s));
+            RMI_TRY(swiglu_cols(e.ug, e.ug + c.n_ff, e.q8f, c.n_ff, nc, 2 * c.n_ff, e.cols, e.s));
     }
     return gemv_res(e, L.down, e.q8f, x, part, nc);
 }
@@ -584,8 +596,15 @@ int attn_block(Engine& e, Layer& L, float* x, float* part, const int* pos, int n
         RMI_TRY(gemv_res(e, L.out_proj, e.q8y, x, part, nc));
         return ffn(e, L, x, part, nc);
     }
-    RMI_TRY(rmi_attn_prep_rope(e.proj, e.q3_rows, L.qn, L.kn, L.kc, L.vc, pos, e.qbuf, c.n_head, c.n_kv, c.head_dim,
-                               c.n_rot, &e.rope, c.eps, nc, e.max_ctx, e.s));
+    RMI_TRY(attn_prep_cols(e.proj, e.q3_rows, L.qn, L.kn, L.kc, L.vc, pos, e.qbuf, c.n_head, c.n_kv, c.head_dim,
+                           c.n_rot, &e.rope, c.eps, nc, e.cols, e.max_ctx, e.s));
+    if (nc > kChunk) {
+        RMI_TRY(flash_wide(e.qbuf, L.kc, L.vc, pos, e.wide_pos, e.proj, e.q3_rows, e.q8y, static_cast<int>(q8y_col),
+                           e.attn_ws, kWideAttnTok, c.n_head, c.n_kv, c.head_dim, nc, e.max_ctx, e.nsub,
+                           1.0f / sqrtf(static_cast<float>(c.head_dim)), e.s));
+        RMI_TRY(gemv_res(e, L.out_proj, e.q8y, x, part, nc));
+        return ffn(e, L, x, part, nc);
+    }
     const int per = std::max(1, kAttnSlots / (c.n_head / c.n_kv));   // tokens per attention launch
     for (int c0 = 0; c0 < nc; c0 += per) {
         RMI_TRY(rmi_gqa_flash_decode(e.qbuf + static_cast<size_t>(c0) * e.attn_q, L.kc, L.vc, pos + c0,
@@ -602,6 +621,13 @@ int gdn_block(Engine& e, Layer& L, int nc) {
     const auto& c = e.cfg;
     RMI_TRY(norm_gemv(e, L.in_proj, e.x, e.part, L.attn_norm, e.proj, nc));
     const int qkvz = 2 * c.ssm_h_k * kS + 2 * c.ssm_h_v * kS;
+    if (nc > kChunk) {
+        RMI_TRY(gdn_wide(L.state[0], L.state[1], L.hist[0], L.hist[1], e.ints + kSel, e.proj, e.qkvz_rows, e.proj + qkvz,
+                         e.qkvz_rows, L.conv_w, L.dt, L.ssm_a, L.ssm_norm, c.eps, e.y, e.q8y,
+                         static_cast<int>(q81_bytes(e.gdn_v)), c.ssm_h_k, c.ssm_h_v, nc, e.gdn_ws, e.s));
+        RMI_TRY(gemv_res(e, L.out_proj, e.q8y, e.x, e.part, nc));
+        return ffn(e, L, e.x, e.part, nc);
+    }
     RMI_TRY(rmi_gdn_layer_tokens_x(L.state[0], L.state[1], L.hist[0], L.hist[1], e.ints + kSel, e.proj, e.qkvz_rows,
                                    e.proj + qkvz, e.qkvz_rows, L.conv_w, L.dt, L.ssm_a, L.ssm_norm, c.eps, e.y, e.gdn_v,
                                    e.q8y, static_cast<int>(q81_bytes(e.gdn_v)), c.ssm_h_k, c.ssm_h_v, nc, e.gdn_xch,
@@ -621,7 +647,7 @@ enum Tail { kTailNone, kTailVerify, kTailSingle };
 int trunk_cols(Engine& e, int nc, const int* tok, const int* pos, float* h, float* hp, Head head,
                Tail tail = kTailNone) {
     const auto& c = e.cfg;
-    RMI_TRY(rmi_embed(e.emb_type, e.tok_embd, tok, e.x, e.part, c.n_embd, c.n_vocab, nc, e.s));
+    RMI_TRY(embed_cols(e.emb_type, e.tok_embd, tok, e.x, e.part, c.n_embd, c.n_vocab, nc, e.cols, e.s));
     const int nl = static_cast<int>(e.layers.size());
     int rope_mode = 1;   // every attention layer of the pass rotates at pos: the first writes the table, the rest read
     for (int il = 0; il < nl; ++il) {
@@ -652,7 +678,7 @@ int trunk_cols(Engine& e, int nc, const int* tok, const int* pos, float* h, floa
         }
         RMI_TRY(rmi_argmax(e.logits, c.n_vocab, ncol, c.n_vocab, e.ints + kV0, e.argmax_ws, e.s));
     }
-    return rmi_rms_norm_out(e.x, e.out_norm, e.part, h, hp, c.n_embd, c.eps, nc, e.s);
+    return rms_norm_out_cols(e.x, e.out_norm, e.part, h, c.n_embd, hp, c.n_embd, c.eps, nc, e.cols, e.s);
 }
 
 // trunk for the decode columns: tokens ints[kTok0 + c] at positions ints[kPos] + c, head on every column
@@ -672,8 +698,8 @@ int draft_cols(Engine& e, const int* tok, const int* pos, const float* h, const 
     const auto& c = e.cfg;
     // [enorm(emb) | hnorm(h)] straight into the Q8_1 row of eh_proj's input, the embedding rows dequantized in the
     // same launch: the bits of embed, norm, norm, quantize
-    RMI_TRY(rmi_embed_quant_apply_pair(e.emb_type, e.tok_embd, tok, e.enorm, h, e.hnorm, hp, e.q8f, c.n_embd,
-                                       c.n_vocab, c.eps, nc, e.s));
+    RMI_TRY(embed_quant_pair_cols(e.emb_type, e.tok_embd, tok, e.enorm, h, e.hnorm, hp, e.q8f, c.n_embd, c.n_vocab,
+                                  c.eps, nc, e.cols, e.s));
     RMI_TRY(gemv(e, e.eh_proj, e.q8f, e.dx, nc));
     // dx's partials: formed by the draft layer's first norm itself (one launch fewer)
     e.norm_self = true;
@@ -705,10 +731,10 @@ int draft_block(Engine& e, const float* h, const float* hp, int nc, bool with_he
 int ingest_chunk(Engine& e, int nc, bool head) {
     const auto& c = e.cfg;
     const size_t np = c.n_embd / 4;
-    hipLaunchKernelGGL(chunk_setup_kernel, dim3(1), dim3(kChunk), 0, e.s, e.ints, e.prompt, e.cints, nc);
+    hipLaunchKernelGGL(chunk_setup_kernel, dim3((nc + 63) / 64), dim3(64), 0, e.s, e.ints, e.prompt, e.cints, e.cols, nc);
     RMI_TRY(launch_status("chunk_setup"));
     const int* tok = e.cints;
-    const int* pos = e.cints + kChunk;
+    const int* pos = e.cints + e.cols;
     RMI_TRY(trunk_cols(e, nc, tok, pos, e.hsave + c.n_embd, e.hpart + np, head ? kHeadLast : kHeadNone));
     RMI_TRY(draft_cols(e, tok, pos, e.hsave, e.hpart, nc, false));
     hipLaunchKernelGGL(chunk_finish_kernel, dim3(1), dim3(256), 0, e.s, e.ints, e.hsave, e.hpart, c.n_embd,
@@ -1151,7 +1177,16 @@ int weights_gguf(Engine& e, const rmi_gguf* g) {
     return RMI_OK;
 }
 
-// round state and activations (kChunk columns), after the weights
+// every matrix of the layers is a packed Q6_K one (the wide chunks' GEMM reads that layout)
+bool wide_capable(const Engine& e) {
+    auto packed = [](const Mat& m) { return m.packed && m.parts.empty(); };
+    auto layer = [&](const Layer& L) { return packed(L.in_proj) && packed(L.out_proj) && packed(L.upgate) && packed(L.down); };
+    for (const auto& L : e.layers)
+        if (!layer(L)) return false;
+    return layer(e.draft) && packed(e.eh_proj) && e.max_ctx > kWideMin;
+}
+
+// round state and activations (cols columns), after the weights
 int alloc_runtime(Engine& e) {
     const auto& c = e.cfg;
     HIP_TRY(hipStreamSynchronize(e.s));   // every pack has read the staging buffer
@@ -1171,7 +1206,9 @@ int alloc_runtime(Engine& e) {
     RMI_TRY(e.alloc(&e.ref_tok, static_cast<size_t>(e.max_ctx) + 1));
     RMI_TRY(e.alloc(&e.pattern, 4096));
     const size_t np = c.n_embd / 4;
-    const size_t K = kChunk;
+    e.wide = wide_capable(e);
+    if (e.wide) e.cols = std::min(kWideCols, e.max_ctx);
+    const size_t K = e.cols;
     RMI_TRY(e.alloc(&e.cints, 2 * K));
     RMI_TRY(e.alloc(&e.prompt, static_cast<size_t>(e.max_ctx)));
     RMI_TRY(e.alloc(&e.x, K * c.n_embd));
@@ -1193,8 +1230,16 @@ int alloc_runtime(Engine& e) {
     RMI_TRY(e.alloc(&e.q8f, K * q81_bytes(e.max_in)));
     RMI_TRY(e.alloc(&e.q8y, K * q81_bytes(std::max(e.gdn_v, e.attn_q))));
     uint8_t* ws = nullptr;
-    RMI_TRY(e.alloc(&ws, rmi_gqa_workspace_bytes(e.max_ctx, c.n_kv, e.nsub)));
+    size_t aws = rmi_gqa_workspace_bytes(e.max_ctx, c.n_kv, e.nsub);
+    if (e.wide) aws = std::max(aws, flash_wide_bytes(e.max_ctx, c.n_head, c.n_kv, e.nsub, kWideAttnTok));
+    RMI_TRY(e.alloc(&ws, aws));
     e.attn_ws = ws;
+    if (e.wide) {
+        RMI_TRY(e.alloc(&ws, ingest_operand_bytes(e.max_in, e.cols)));
+        e.gemm_ws = ws;
+        RMI_TRY(e.alloc(&ws, gdn_wide_bytes(c.ssm_h_k, c.ssm_h_v, e.cols)));
+        e.gdn_ws = ws;
+    }
     RMI_TRY(e.alloc(&e.rope_cs, rmi_gqa_rope_table_bytes(c.n_rot) / sizeof(float)));
     uint8_t* aw = nullptr;
     RMI_TRY(e.alloc(&aw, rmi_argmax_workspace_bytes(2)));
@@ -1397,7 +1442,16 @@ extern "C" int rmi_engine_ingest(rmi_engine* h, const int* tokens, int n, int ba
         HIP_TRY(hipMemcpyAsync(e.prompt + pos0, tokens, sizeof(int) * static_cast<size_t>(n), hipMemcpyHostToDevice,
                                e.s));
         int i = 0;
-        if (batch == kChunk && n > kChunk) {
+        // the largest batch: wide chunks while enough tokens are left (the same state, fewer passes over the weights)
+        if (batch == kChunk && e.wide) {
+            while (n - i >= kWideMin) {
+                const int nc = std::min(e.cols, n - i);
+                e.wide_pos = pos0 + i;
+                RMI_TRY(ingest_chunk(e, nc, i + nc == n));
+                i += nc;
+            }
+        }
+        if (batch == kChunk && n - i > kChunk) {
             RMI_TRY(capture(e, &e.g_chunk, [&] { return ingest_chunk(e, kChunk, false); }));
             for (; n - i > kChunk; i += kChunk) HIP_TRY(hipGraphLaunch(e.g_chunk, e.s));
         }

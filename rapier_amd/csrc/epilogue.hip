@@ -6,6 +6,7 @@
 //
 // Norm reduction (rms_quant_apply / rms_norm_out): 256 lanes; lane t adds partials t, t+256, t+512, ... in order,
 // then a 64-lane xor butterfly, then the 4 wave sums in order.  Every workgroup derives the same bits.
+#include "ingest.h"
 #include "epilogue_dev.h"
 
 namespace rmi {
@@ -272,31 +273,41 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint8_t* __restrict__ 
     }
 }
 
-bool bad_cols(int ncols) { return ncols < 1 || ncols > kMaxCols; }
+bool bad_cols(int ncols, int limit = kMaxCols) { return ncols < 1 || ncols > limit; }
 
 }  // namespace
 }  // namespace rmi
 
 using namespace rmi;
 
-extern "C" int rmi_rms_quant_apply(const float* x, const float* w, const float* partials, void* y_q8_1, int cols,
-                                   float eps, int ncols, void* stream) {
-    if (cols <= 0 || cols % 32 != 0 || bad_cols(ncols)) return fail(RMI_ERR_SHAPE, "rms_quant_apply: bad shape");
+int rmi::rms_quant_cols(const float* x, const float* w, const float* partials, void* y_q8_1, int cols, float eps,
+                        int ncols, int limit, hipStream_t stream) {
+    if (cols <= 0 || cols % 32 != 0 || bad_cols(ncols, limit)) return fail(RMI_ERR_SHAPE, "rms_quant_apply: bad shape");
     if (!aligned4(x) || !aligned4(w) || !aligned4(partials) || !aligned4(y_q8_1))
         return fail(RMI_ERR_POINTER, "rms_quant_apply: null or misaligned pointer");
     hipLaunchKernelGGL(rms_quant_apply_kernel, dim3((cols + 255) / 256, ncols), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), x, w, partials, static_cast<uint8_t*>(y_q8_1), cols, eps);
+                       stream, x, w, partials, static_cast<uint8_t*>(y_q8_1), cols, eps);
     return launch_status("rms_quant_apply");
+}
+
+extern "C" int rmi_rms_quant_apply(const float* x, const float* w, const float* partials, void* y_q8_1, int cols,
+                                   float eps, int ncols, void* stream) {
+    return rms_quant_cols(x, w, partials, y_q8_1, cols, eps, ncols, kMaxCols, static_cast<hipStream_t>(stream));
+}
+
+int rmi::rms_quant_self_cols(const float* x, const float* w, void* y_q8_1, int cols, float eps, int ncols, int limit,
+                             hipStream_t stream) {
+    if (cols <= 0 || cols % 32 != 0 || bad_cols(ncols, limit)) return fail(RMI_ERR_SHAPE, "rms_quant_apply_self: bad shape");
+    if (!aligned16(x) || !aligned4(w) || !aligned4(y_q8_1))
+        return fail(RMI_ERR_POINTER, "rms_quant_apply_self: null or misaligned pointer");
+    hipLaunchKernelGGL(rms_quant_self_kernel, dim3((cols + 255) / 256, ncols), dim3(256), 0,
+                       stream, x, w, static_cast<uint8_t*>(y_q8_1), cols, eps);
+    return launch_status("rms_quant_apply_self");
 }
 
 extern "C" int rmi_rms_quant_apply_self(const float* x, const float* w, void* y_q8_1, int cols, float eps, int ncols,
                                         void* stream) {
-    if (cols <= 0 || cols % 32 != 0 || bad_cols(ncols)) return fail(RMI_ERR_SHAPE, "rms_quant_apply_self: bad shape");
-    if (!aligned16(x) || !aligned4(w) || !aligned4(y_q8_1))
-        return fail(RMI_ERR_POINTER, "rms_quant_apply_self: null or misaligned pointer");
-    hipLaunchKernelGGL(rms_quant_self_kernel, dim3((cols + 255) / 256, ncols), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), x, w, static_cast<uint8_t*>(y_q8_1), cols, eps);
-    return launch_status("rms_quant_apply_self");
+    return rms_quant_self_cols(x, w, y_q8_1, cols, eps, ncols, kMaxCols, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rmi_rms_quant_apply_pair(const float* x0, const float* w0, const float* partials0, const float* x1,
@@ -312,16 +323,22 @@ extern "C" int rmi_rms_quant_apply_pair(const float* x0, const float* w0, const 
     return launch_status("rms_quant_apply_pair");
 }
 
-extern "C" int rmi_rms_norm_out_strided(const float* x, const float* w, const float* partials, float* out,
-                                        int out_stride, float* out_partials, int cols, float eps, int ncols,
-                                        void* stream) {
-    if (cols <= 0 || cols % 4 != 0 || bad_cols(ncols) || out_stride < cols)
+int rmi::rms_norm_out_cols(const float* x, const float* w, const float* partials, float* out, int out_stride,
+                           float* out_partials, int cols, float eps, int ncols, int limit, hipStream_t stream) {
+    if (cols <= 0 || cols % 4 != 0 || bad_cols(ncols, limit) || out_stride < cols)
         return fail(RMI_ERR_SHAPE, "rms_norm_out: bad shape");
     if (!aligned4(x) || !aligned4(w) || !aligned4(partials) || !aligned4(out))
         return fail(RMI_ERR_POINTER, "rms_norm_out: null or misaligned pointer");
     hipLaunchKernelGGL(rms_norm_out_kernel, dim3((cols + 255) / 256, ncols), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), x, w, partials, out, out_partials, cols, eps, out_stride);
+                       stream, x, w, partials, out, out_partials, cols, eps, out_stride);
     return launch_status("rms_norm_out");
+}
+
+extern "C" int rmi_rms_norm_out_strided(const float* x, const float* w, const float* partials, float* out,
+                                        int out_stride, float* out_partials, int cols, float eps, int ncols,
+                                        void* stream) {
+    return rms_norm_out_cols(x, w, partials, out, out_stride, out_partials, cols, eps, ncols, kMaxCols,
+                             static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rmi_rms_norm_out(const float* x, const float* w, const float* partials, float* out, float* out_partials,
@@ -347,23 +364,33 @@ extern "C" int rmi_add_partials(float* x, const float* o, float* partials, int n
     return launch_status("add_partials");
 }
 
-extern "C" int rmi_swiglu_quant_interleaved(const float* up_gate, void* y_q8_1, int n, int ncols, int col_stride,
-                                            void* stream) {
-    if (n <= 0 || n % 32 != 0 || bad_cols(ncols) || col_stride < 2 * n)
+int rmi::swiglu_interleaved_cols(const float* up_gate, void* y_q8_1, int n, int ncols, int col_stride, int limit,
+                                 hipStream_t stream) {
+    if (n <= 0 || n % 32 != 0 || bad_cols(ncols, limit) || col_stride < 2 * n)
         return fail(RMI_ERR_SHAPE, "swiglu_quant_interleaved: bad shape");
     if (!aligned4(up_gate) || !aligned4(y_q8_1)) return fail(RMI_ERR_POINTER, "swiglu_quant_interleaved: bad pointer");
     hipLaunchKernelGGL(swiglu_quant_interleaved_kernel, dim3((n + 255) / 256, ncols), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), up_gate, static_cast<uint8_t*>(y_q8_1), n, col_stride);
+                       stream, up_gate, static_cast<uint8_t*>(y_q8_1), n, col_stride);
     return launch_status("swiglu_quant_interleaved");
+}
+
+extern "C" int rmi_swiglu_quant_interleaved(const float* up_gate, void* y_q8_1, int n, int ncols, int col_stride,
+                                            void* stream) {
+    return swiglu_interleaved_cols(up_gate, y_q8_1, n, ncols, col_stride, kMaxCols, static_cast<hipStream_t>(stream));
+}
+
+int rmi::swiglu_cols(const float* up, const float* gate, void* y_q8_1, int n, int ncols, int col_stride, int limit,
+                     hipStream_t stream) {
+    if (n <= 0 || n % 32 != 0 || bad_cols(ncols, limit) || col_stride < n) return fail(RMI_ERR_SHAPE, "swiglu_quant: bad shape");
+    if (!aligned4(up) || !aligned4(gate) || !aligned4(y_q8_1)) return fail(RMI_ERR_POINTER, "swiglu_quant: null pointer");
+    hipLaunchKernelGGL(swiglu_quant_kernel, dim3((n + 255) / 256, ncols), dim3(256), 0,
+                       stream, up, gate, static_cast<uint8_t*>(y_q8_1), n, col_stride);
+    return launch_status("swiglu_quant");
 }
 
 extern "C" int rmi_swiglu_quant(const float* up, const float* gate, void* y_q8_1, int n, int ncols, int col_stride,
                                 void* stream) {
-    if (n <= 0 || n % 32 != 0 || bad_cols(ncols) || col_stride < n) return fail(RMI_ERR_SHAPE, "swiglu_quant: bad shape");
-    if (!aligned4(up) || !aligned4(gate) || !aligned4(y_q8_1)) return fail(RMI_ERR_POINTER, "swiglu_quant: null pointer");
-    hipLaunchKernelGGL(swiglu_quant_kernel, dim3((n + 255) / 256, ncols), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), up, gate, static_cast<uint8_t*>(y_q8_1), n, col_stride);
-    return launch_status("swiglu_quant");
+    return swiglu_cols(up, gate, y_q8_1, n, ncols, col_stride, kMaxCols, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rmi_sig_mul_quant(const float* o, const float* g, void* y_q8_1, int n, int ncols, int o_stride,
@@ -450,10 +477,10 @@ __global__ __launch_bounds__(256) void embed_quant_pair_kernel(const uint8_t* __
     q8_1_store_lane((v * wv) * inv, yc + static_cast<size_t>(i / 32) * kQ8_1Bytes);
 }
 
-extern "C" int rmi_embed_quant_apply_pair(int type, const void* emb, const int* tokens, const float* w0,
-                                          const float* x1, const float* w1, const float* partials1, void* y_q8_1,
-                                          int cols, int n_vocab, float eps, int ncols, void* stream) {
-    if (cols <= 0 || cols % 256 != 0 || n_vocab <= 0 || bad_cols(ncols))
+int rmi::embed_quant_pair_cols(int type, const void* emb, const int* tokens, const float* w0, const float* x1,
+                               const float* w1, const float* partials1, void* y_q8_1, int cols, int n_vocab, float eps,
+                               int ncols, int limit, hipStream_t s) {
+    if (cols <= 0 || cols % 256 != 0 || n_vocab <= 0 || bad_cols(ncols, limit))
         return fail(RMI_ERR_SHAPE, "embed_quant_apply_pair: bad shape");
     if (type != 14 && type != 13 && type != 12) return fail(RMI_ERR_UNSUPPORTED, "embed_quant_apply_pair: type");
     if (!emb || !aligned4(tokens) || !aligned4(w0) || !aligned4(x1) || !aligned4(w1) || !aligned4(partials1) ||
@@ -462,7 +489,6 @@ extern "C" int rmi_embed_quant_apply_pair(int type, const void* emb, const int* 
     const auto* e = static_cast<const uint8_t*>(emb);
     auto* y = static_cast<uint8_t*>(y_q8_1);
     const dim3 grid(cols / 256, ncols, 2), block(256);
-    const hipStream_t s = static_cast<hipStream_t>(stream);
     const NormInput b{x1, w1, partials1};
     if (type == 14) hipLaunchKernelGGL(embed_quant_pair_kernel<14>, grid, block, 0, s, e, tokens, w0, b, y, cols, n_vocab, eps);
     else if (type == 13) hipLaunchKernelGGL(embed_quant_pair_kernel<13>, grid, block, 0, s, e, tokens, w0, b, y, cols, n_vocab, eps);
@@ -470,20 +496,32 @@ extern "C" int rmi_embed_quant_apply_pair(int type, const void* emb, const int* 
     return launch_status("embed_quant_apply_pair");
 }
 
-extern "C" int rmi_embed(int type, const void* emb, const int* tokens, float* x, float* partials, int n_embd,
-                         int n_vocab, int ncols, void* stream) {
-    if (n_embd <= 0 || n_embd % 256 != 0 || n_vocab <= 0 || bad_cols(ncols))
+extern "C" int rmi_embed_quant_apply_pair(int type, const void* emb, const int* tokens, const float* w0,
+                                          const float* x1, const float* w1, const float* partials1, void* y_q8_1,
+                                          int cols, int n_vocab, float eps, int ncols, void* stream) {
+    return embed_quant_pair_cols(type, emb, tokens, w0, x1, w1, partials1, y_q8_1, cols, n_vocab, eps, ncols, kMaxCols,
+                                 static_cast<hipStream_t>(stream));
+}
+
+int rmi::embed_cols(int type, const void* emb, const int* tokens, float* x, float* partials, int n_embd, int n_vocab,
+                    int ncols, int limit, hipStream_t s) {
+    if (n_embd <= 0 || n_embd % 256 != 0 || n_vocab <= 0 || bad_cols(ncols, limit))
         return fail(RMI_ERR_SHAPE, "embed: bad shape");
     if (type != 14 && type != 13 && type != 12) return fail(RMI_ERR_UNSUPPORTED, "embed: token_embd type must be Q6_K, Q5_K or Q4_K");
     if (!emb || !aligned4(tokens) || !aligned4(x) || !aligned4(partials))
         return fail(RMI_ERR_POINTER, "embed: null or misaligned pointer");
-    const auto s = static_cast<hipStream_t>(stream);
     const dim3 grid(n_embd / 256, ncols), block(256);
     const auto* e = static_cast<const uint8_t*>(emb);
     if (type == 14) hipLaunchKernelGGL(embed_kernel<14>, grid, block, 0, s, e, tokens, x, partials, n_embd, n_vocab);
     else if (type == 13) hipLaunchKernelGGL(embed_kernel<13>, grid, block, 0, s, e, tokens, x, partials, n_embd, n_vocab);
     else hipLaunchKernelGGL(embed_kernel<12>, grid, block, 0, s, e, tokens, x, partials, n_embd, n_vocab);
     return launch_status("embed");
+}
+
+extern "C" int rmi_embed(int type, const void* emb, const int* tokens, float* x, float* partials, int n_embd,
+                         int n_vocab, int ncols, void* stream) {
+    return embed_cols(type, emb, tokens, x, partials, n_embd, n_vocab, ncols, kMaxCols,
+                      static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rmi_embed_q6_k(const void* emb, const int* tokens, float* x, float* partials, int n_embd, int n_vocab,

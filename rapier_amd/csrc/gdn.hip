@@ -18,6 +18,7 @@
 // live one.  A verify writes the after-token-0 state/history into the other buffer, so rejecting the draft is a flip
 // of `sel` (no copy).  A single-token step updates the live buffers in place.
 #include "rmi_common.h"
+#include "ingest.h"
 
 namespace rmi {
 namespace {
@@ -704,7 +705,231 @@ __global__ __launch_bounds__(kPartLanes) void gdn_split_kernel(StepArgs a) {
     }
 }
 
+
+// ---- wide ingest chunks: conv, recurrence and output norm as three launches -------------------------------------------
+// Only the recurrence is serial in the tokens.  (1) gdn_wide_prep runs the conv + SiLU + L2 and the gates of every token
+// in parallel; (2) gdn_wide_scan walks the tokens with one wave per 16 columns of a value head, the state in its
+// registers, and leaves the raw outputs and the waves' sums of squares; (3) gdn_wide_finish takes the output norm, the
+// gate and the Q8_1 blocks.  Lane ownership, expressions and reduction orders are gdn_step_kernel's (a wave there is a
+// wave here), so the bits are those of the per-token steps.
+// The scan is bound by its own vector instructions, 128 per token and lane (mul, two fmas of the update and output, one
+// fma of the next token's S^T k, which rides along so that the two chains hide each other's latency); 256 waves of the
+// 9B shape, one per CU.  1000 tokens of a 9B layer: 608 us (prep 17, scan 574, finish 17) where 62.5 launches of the
+// 16-token kernel take 1410 us.
+constexpr int kScanTok = 16;   // tokens staged per step, double-buffered
+
+struct WideArgs {
+    StepArgs a;
+    float* qk;     // [token][h_k][q 128 | k 128], convolved and normalized
+    float* v;      // [token][h_v][128], convolved
+    float* gb;     // [h_v][tpad][decay, beta]
+    float* wsum;   // [token][h_v][8]
+    int tpad;      // tokens of gb's rows, a multiple of 32
+};
+
+constexpr int kPrepTok = 8;
+
+__global__ __launch_bounds__(S) void gdn_wide_prep(WideArgs w) {
+    const StepArgs& a = w.a;
+    __shared__ float cpart[kPrepTok][2];
+    const int id = blockIdx.x, t0 = static_cast<int>(blockIdx.y) * kPrepTok, j = threadIdx.x;
+    const int nt = min(kPrepTok, a.ntok - t0);
+    if (id == 2 * a.h_k + a.h_v) {   // the gates
+        for (int i = j; i < nt * a.h_v; i += S) {
+            const int t = t0 + i / a.h_v, h = i % a.h_v;
+            const float* ab = a.ab + static_cast<size_t>(t) * a.ab_stride;
+            float g, b;
+            gate_values(ab[h], ab[a.h_v + h], a.dt[h], a.ssm_a[h], g, b);
+            reinterpret_cast<float2*>(w.gb)[static_cast<size_t>(h) * w.tpad + t] = make_float2(g, b);
+        }
+        return;
+    }
+    const int kind = id < a.h_k ? 0 : id < 2 * a.h_k ? 1 : 2;
+    const int head = kind == 0 ? id : kind == 1 ? id - a.h_k : id - 2 * a.h_k;
+    const float* src = (kind == 0 ? a.q : kind == 1 ? a.k : a.v) + head * S + j;
+    const int c = (kind == 2 ? 2 * a.h_k : kind * a.h_k) * S + head * S + j;
+    const bool sel_b = *a.sel != 0;
+    const float* hist = (sel_b ? a.hist_b : a.hist_a) + 3 * ((3 * head + kind) * S + j);
+    float x[kPrepTok + 3];
+#pragma unroll
+    for (int i = 0; i < kPrepTok + 3; ++i) {
+        const int t = t0 + i - 3;
+        const float xv = src[static_cast<size_t>(min(max(t, 0), a.ntok - 1)) * a.tok_stride];
+        x[i] = t < 0 ? hist[min(t + 3, 2)] : xv;
+    }
+    const float w0 = a.conv_w[4 * c], w1 = a.conv_w[4 * c + 1], w2 = a.conv_w[4 * c + 2], w3 = a.conv_w[4 * c + 3];
+    float y[kPrepTok];
+#pragma unroll
+    for (int t = 0; t < kPrepTok; ++t)
+        y[t] = silu(__builtin_fmaf(x[t + 3], w3, __builtin_fmaf(x[t + 2], w2, __builtin_fmaf(x[t + 1], w1, x[t] * w0))));
+    if (kind < 2) {   // uniform
+#pragma unroll
+        for (int t = 0; t < kPrepTok; ++t) {
+            const float sqs = group_sum<64>(y[t] * y[t]);
+            if ((j & 63) == 0) cpart[t][j >> 6] = sqs;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kPrepTok; ++t) y[t] *= rsqrtf((cpart[t][0] + cpart[t][1]) + a.eps);
+    }
+    float* dst = kind == 2 ? w.v + (static_cast<size_t>(t0) * a.h_v + head) * S + j
+                           : w.qk + (static_cast<size_t>(t0) * a.h_k + head) * 2 * S + kind * S + j;
+    const size_t stride = kind == 2 ? static_cast<size_t>(a.h_v) * S : static_cast<size_t>(a.h_k) * 2 * S;
+#pragma unroll
+    for (int t = 0; t < kPrepTok; ++t)
+        if (t < nt) dst[t * stride] = y[t];
+}
+
+__device__ __forceinline__ void scan_to_lds(const float* g, float* l, bool wide) {
+    if (wide)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) g,
+                                         (__attribute__((address_space(3))) void*) l, 16, 0, 0);
+    else
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) g,
+                                         (__attribute__((address_space(3))) void*) l, 4, 0, 0);
+}
+
+__global__ __launch_bounds__(64) void gdn_wide_scan(WideArgs w) {
+    const StepArgs& a = w.a;
+    __shared__ __attribute__((aligned(16))) float sqk[2][kScanTok][2 * S];
+    __shared__ __attribute__((aligned(16))) float sv[2][kScanTok][16];
+    __shared__ __attribute__((aligned(16))) float sgb[2][2 * kScanTok][2];
+    __shared__ __attribute__((aligned(16))) float so[kScanTok][16];
+    __shared__ float sw[kScanTok];
+    // workgroup w * h_v + head: round robin over the XCDs, so a head's eight waves (h_v a multiple of 8) share an L2
+    const int head = static_cast<int>(blockIdx.x) % a.h_v, wv = static_cast<int>(blockIdx.x) / a.h_v;
+    const int ln = threadIdx.x, rg = ln >> 4;
+    const int col = 16 * wv + (ln & 15);
+    const int qh = head % a.h_k;
+    const size_t row_stride = static_cast<size_t>(a.h_v) * S;
+    const size_t base = (static_cast<size_t>(rg * RPG) * a.h_v + head) * S + col;
+    const bool sel_b = *a.sel != 0;
+    float* state = sel_b ? a.state_b : a.state_a;
+    float* hist = sel_b ? a.hist_b : a.hist_a;
+    float s[RPG];
+#pragma unroll
+    for (int r = 0; r < RPG; ++r) s[r] = state[base + r * row_stride];
+    // tokens t0 .. t0 + 15 into buffer b (the buffers are padded to whole steps: rows past the last are not used)
+    auto fetch = [&](int t0, int b) {
+#pragma unroll
+        for (int t = 0; t < kScanTok; ++t)
+            scan_to_lds(w.qk + (static_cast<size_t>(t0 + t) * a.h_k + qh) * 2 * S + 4 * ln, sqk[b][t], true);
+        scan_to_lds(w.v + (static_cast<size_t>(t0 + (ln >> 2)) * a.h_v + head) * S + 16 * wv + 4 * (ln & 3), sv[b][0], true);
+        scan_to_lds(w.gb + (static_cast<size_t>(head) * w.tpad + t0) * 2 + ln, sgb[b][0], false);
+    };
+    fetch(0, 0);
+    // this wave's channels of the conv history become the last three inputs (gdn_wide_prep has read the old ones)
+    if (ln < 48) {
+        const int kind = ln >> 4;
+        const float* src = (kind == 0 ? a.q + qh * S : kind == 1 ? a.k + qh * S : a.v + head * S) + col;
+        float* dst = hist + 3 * ((3 * head + kind) * S + col);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) dst[i] = src[static_cast<size_t>(a.ntok - 3 + i) * a.tok_stride];
+    }
+    for (int t0 = 0, b = 0; t0 < a.ntok; t0 += kScanTok, b ^= 1) {
+        // this step's tokens have arrived, and the stores of the previous step are out
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        const int nt = min(kScanTok, a.ntok - t0);
+        if (t0 + kScanTok < a.ntok) fetch(t0 + kScanTok, b ^ 1);
+        float k[RPG], kv = 0.0f;
+#pragma unroll
+        for (int r4 = 0; r4 < RPG / 4; ++r4)
+            *reinterpret_cast<float4*>(k + 4 * r4) = *reinterpret_cast<const float4*>(&sqk[b][0][S + rg * RPG + 4 * r4]);
+#pragma unroll
+        for (int r = 0; r < RPG; ++r) kv = __builtin_fmaf(s[r], k[r], kv);
+        for (int t = 0; t < nt; ++t) {
+            float q[RPG], kn[RPG];
+            const int tn = min(t + 1, kScanTok - 1);
+#pragma unroll
+            for (int r4 = 0; r4 < RPG / 4; ++r4) {
+                *reinterpret_cast<float4*>(q + 4 * r4) = *reinterpret_cast<const float4*>(&sqk[b][t][rg * RPG + 4 * r4]);
+                *reinterpret_cast<float4*>(kn + 4 * r4) =
+                    *reinterpret_cast<const float4*>(&sqk[b][tn][S + rg * RPG + 4 * r4]);
+            }
+            const float g = sgb[b][t][0], beta = sgb[b][t][1];
+            const float vcol = sv[b][t][ln & 15];
+            kv = sum_row_groups(kv);
+            const float delta = (vcol - g * kv) * beta;
+            float o = 0.0f, kvn = 0.0f;
+#pragma unroll
+            for (int r = 0; r < RPG; ++r) {
+                s[r] = __builtin_fmaf(g, s[r], k[r] * delta);
+                o = __builtin_fmaf(s[r], q[r], o);
+                kvn = __builtin_fmaf(s[r], kn[r], kvn);
+            }
+            o = sum_row_groups(o);
+            const float oc = o * 0.08838834764831845f;   // 1 / sqrt(128)
+            const float ss = group_sum<16>(oc * oc);
+            if (rg == 0) so[t][ln] = oc;
+            if (ln == 0) sw[t] = ss;
+            kv = kvn;
+#pragma unroll
+            for (int r = 0; r < RPG; ++r) k[r] = kn[r];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const int tt = ln >> 2;
+        if (tt < nt)
+            *reinterpret_cast<float4*>(a.y + static_cast<size_t>(t0 + tt) * a.y_stride + head * S + 16 * wv + 4 * (ln & 3)) =
+                *reinterpret_cast<const float4*>(&so[tt][4 * (ln & 3)]);
+        if (ln < nt) w.wsum[(static_cast<size_t>(t0 + ln) * a.h_v + head) * 8 + wv] = sw[ln];
+    }
+#pragma unroll
+    for (int r = 0; r < RPG; ++r) state[base + r * row_stride] = s[r];
+}
+
+__global__ __launch_bounds__(2 * S) void gdn_wide_finish(WideArgs w) {
+    const StepArgs& a = w.a;
+    const int t = blockIdx.y, head = static_cast<int>(blockIdx.x) * 2 + (threadIdx.x >> 7), col = threadIdx.x & (S - 1);
+    if (head >= a.h_v) return;   // whole waves
+    float* y = a.y + static_cast<size_t>(t) * a.y_stride + head * S + col;
+    const float occ = *y;
+    const float zz = a.z[static_cast<size_t>(t) * a.tok_stride + head * S + col];
+    const float gam = a.gamma[col];
+    const float* ws = w.wsum + (static_cast<size_t>(t) * a.h_v + head) * 8;
+    float tot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < S * RG / 64; ++i) tot += ws[i];
+    const float scl = rsqrtf(tot / static_cast<float>(S) + a.eps);
+    const float yv = occ * scl * gam * silu(zz);
+    *y = yv;
+    q8_1_store_lane(yv, a.q8 + static_cast<size_t>(t) * a.q8_stride + (head * 4 + (col >> 5)) * kQ8_1Bytes);
+}
+
+int wide_tok(int ntok) { return (ntok + 31) / 32 * 32; }
+
 }  // namespace
+
+size_t gdn_wide_bytes(int h_k, int h_v, int ntok) {
+    return static_cast<size_t>(wide_tok(ntok)) * (2 * h_k * S + h_v * S + 2 * h_v + 8 * h_v) * sizeof(float);
+}
+
+int gdn_wide(float* state_a, float* state_b, float* hist_a, float* hist_b, const int* sel, const float* qkvz,
+             int stride, const float* ab, int ab_stride, const float* conv_w, const float* dt, const float* ssm_a,
+             const float* gamma, float eps, float* y, uint8_t* q8, int q8_stride, int h_k, int h_v, int ntok, void* ws,
+             hipStream_t s) {
+    if (h_k <= 0 || h_v <= 0 || h_v % h_k || ntok < 3 || !aligned16(y) || !aligned16(ws) || !q8)
+        return fail(RMI_ERR_SHAPE, "gdn_wide: invalid arguments");
+    WideArgs w{};
+    StepArgs& a = w.a;
+    a.state_a = state_a; a.state_b = state_b; a.sel = sel;
+    a.q = qkvz; a.k = qkvz + h_k * S; a.v = qkvz + 2 * h_k * S; a.z = qkvz + 2 * h_k * S + h_v * S;
+    a.tok_stride = stride;
+    a.ab = ab; a.ab_stride = ab_stride; a.dt = dt; a.ssm_a = ssm_a;
+    a.gamma = gamma; a.eps = eps;
+    a.y = y; a.y_stride = h_v * S; a.q8 = q8; a.q8_stride = q8_stride;
+    a.h_k = h_k; a.h_v = h_v;
+    a.hist_a = hist_a; a.hist_b = hist_b; a.conv_w = conv_w;
+    a.ntok = ntok;
+    w.tpad = wide_tok(ntok);
+    w.qk = static_cast<float*>(ws);
+    w.v = w.qk + static_cast<size_t>(w.tpad) * 2 * h_k * S;
+    w.gb = w.v + static_cast<size_t>(w.tpad) * h_v * S;
+    w.wsum = w.gb + static_cast<size_t>(w.tpad) * 2 * h_v;
+    hipLaunchKernelGGL(gdn_wide_prep, dim3(2 * h_k + h_v + 1, (ntok + kPrepTok - 1) / kPrepTok), dim3(S), 0, s, w);
+    hipLaunchKernelGGL(gdn_wide_scan, dim3(h_v * (S / 16)), dim3(64), 0, s, w);
+    hipLaunchKernelGGL(gdn_wide_finish, dim3((h_v + 1) / 2, ntok), dim3(2 * S), 0, s, w);
+    return launch_status("gdn_wide");
+}
 }  // namespace rmi
 
 using namespace rmi;
