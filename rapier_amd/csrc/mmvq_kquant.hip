@@ -220,6 +220,9 @@ int launch(const void* wv, const void* xv, float* y, const float* res, float* pa
            hipStream_t s) {
     const auto* w = static_cast<const uint8_t*>(wv);
     const auto* x = static_cast<const uint8_t*>(xv);
+    if (ncols > 2)
+        if (const int rc = cols_gemv(TYPE, 64, w, x, y, res, partials, n_in, n_out, ncols, s); rc >= 0)
+            return rc;
     const int per = std::max(1, std::min(4, kStageMax / ((n_in / 32) * 40)));
     const size_t xcol = static_cast<size_t>(n_in / 32) * kQ8_1Bytes;
     const size_t pcol = static_cast<size_t>((n_out + 3) / 4);

@@ -460,6 +460,11 @@ int cu_count() {
     return n;
 }
 
+bool stream_on() {
+    static const bool on = env_int("RMI_GGUF_STREAM", 1) != 0;
+    return on;
+}
+
 TileCfg pick_cfg(int n_in, int n_out, const void* w) {
     static const int depth = env_int("RMI_GEMV_DEPTH", 1);
     static const int per_cu = env_int("RMI_GEMV_PER_CU", 3);
@@ -487,6 +492,18 @@ void launch_depth(const uint8_t* w, const uint8_t* x, float* y, const float* res
     else launch_tiled<R, NCOLS, RES, 2, XM>(w, x, y, res, partials, n_in, n_out, cfg.per_cu, s);
 }
 
+// the lanes the one-column kernel of a shape splits a row's half-blocks over: the stream and 16-row tiled kernels 16, the
+// 8-row one 32, the generic one 64
+bool stream_shape(int n_in, const void* w) {
+    const int nch = n_in / 2048;
+    return n_in % 2048 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 && (nch == 2 || nch == 4 || nch == 6);
+}
+int row_lanes(int n_in, int n_out, const void* w) {
+    if (stream_on() && stream_shape(n_in, w)) return 16;
+    const int rows = pick_cfg(n_in, n_out, w).rows;
+    return rows == 16 ? 16 : rows == 8 ? 32 : 64;
+}
+
 // whole-row staging for rows of at most kFullMaxIn elements (shape-only choice; the staged values are the same)
 bool full_row(int n_in) {
     static const bool on = env_int("RMI_GEMV_XFULL", 1) != 0;
@@ -498,8 +515,7 @@ void launch_cols(const uint8_t* w, const uint8_t* x, float* y, const float* res,
                  hipStream_t s) {
     // rows of 4096 / 8192 / 12288: the stream kernel (every column, including the passes of ncols > 4, bitwise its
     // one-column result and the packed kernels'); RMI_GGUF_STREAM=0 measures the tiled kernel instead
-    static const bool stream_on = env_int("RMI_GGUF_STREAM", 1) != 0;
-    if (NCOLS <= 4 && stream_on &&
+    if (NCOLS <= 4 && stream_on() &&
         gguf_stream_gemv(w, x, y, RES ? res : nullptr, RES ? partials : nullptr, n_in, n_out, NCOLS, s) == RMI_OK)
         return;
     const TileCfg cfg = pick_cfg(n_in, n_out, w);
@@ -521,6 +537,9 @@ int launch(const void* wv, const void* xv, float* y, const float* res, float* pa
            int ncols, hipStream_t s) {
     const auto* w = static_cast<const uint8_t*>(wv);
     const auto* x = static_cast<const uint8_t*>(xv);
+    if (ncols > 2)
+        if (const int rc = cols_gemv(14, row_lanes(n_in, n_out, w), w, x, y, res, partials, n_in, n_out, ncols, s); rc >= 0)
+            return rc;
     switch (ncols) {
         case 1: launch_cols<1, RES>(w, x, y, res, partials, n_in, n_out, s); break;
         case 2: launch_cols<2, RES>(w, x, y, res, partials, n_in, n_out, s); break;

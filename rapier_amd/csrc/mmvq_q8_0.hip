@@ -72,6 +72,9 @@ int launch(const void* wv, const void* xv, float* y, const float* res, float* pa
     const auto* w = static_cast<const uint8_t*>(wv);
     const auto* x = static_cast<const uint8_t*>(xv);
     const dim3 grid((n_out + 3) / 4), block(256);
+    if (ncols > 2)
+        if (const int rc = cols_gemv(8, 64, w, x, y, res, partials, n_in, n_out, ncols, s); rc >= 0)
+            return rc;
     if (ncols > 4) {
         const size_t xcol = static_cast<size_t>(n_in / 32) * kQ8_1Bytes;
         const size_t pcol = static_cast<size_t>((n_out + 3) / 4);

@@ -177,4 +177,10 @@ int registry_mmvq(const void* w, const void* x_q8_1, float* y, const float* res,
 int gguf_stream_gemv(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials, int n_in,
                      int n_out, int ncols, hipStream_t s);
 
+// GGUF-layout GEMV of up to 16 columns in one weight pass (mmvq_cols.hip), bitwise the one-column kernels'; lanes: the
+// lanes a Q6_K row's half-blocks are split over (16, 32 or 64).  Returns -1, launching nothing, where the narrow passes
+// are faster (few columns) or it does not apply (rows above 12288, lanes 32).
+int cols_gemv(int type, int lanes, const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials,
+              int n_in, int n_out, int ncols, hipStream_t s);
+
 }  // namespace rmi
