@@ -706,6 +706,223 @@ __global__ __launch_bounds__(kPartLanes) void gdn_split_kernel(StepArgs a) {
 }
 
 
+// ---- the recurrence over staged tokens ---------------------------------------------------------------------------------
+// One wave, 16 columns of a value head (lane: column l % 16, row group l / 16, the state's 32 rows in s).  Per token and
+// row: the update's multiply and fma, the output's fma and the next token's S^T k, whose chain hides the output's (128
+// vector instructions per token).  Each lane's share of the output goes to part[token][lane]; the row groups are added
+// and squared for all tokens together afterwards (scan_outputs), off the recurrence's path.  The operations and their
+// order are gdn_step_kernel's.
+struct ScanToken {
+    const float* q;    // the token's q and k rows (128 floats each) in LDS
+    const float* k;
+    float g, beta, v;  // decay, beta, the column's v
+};
+
+template <typename Get>
+__device__ __forceinline__ void scan_tokens(float (&s)[RPG], int nt, int rg, float* part, Get&& get) {
+    auto row = [&](const float* p, float (&r)[RPG]) {
+#pragma unroll
+        for (int i = 0; i < RPG / 4; ++i)
+            *reinterpret_cast<float4*>(r + 4 * i) = *reinterpret_cast<const float4*>(p + rg * RPG + 4 * i);
+    };
+    float ka[RPG], kb[RPG], q[RPG];
+    float kv = 0.0f;
+    row(get(0).k, ka);
+#pragma unroll
+    for (int r = 0; r < RPG; ++r) kv = __builtin_fmaf(s[r], ka[r], kv);
+    // token t with its k row and the next token's (the last token's again behind it, its sum unused)
+    auto step = [&](int t, const float (&k)[RPG], float (&kn)[RPG]) {
+        const ScanToken tk = get(t);
+        row(tk.q, q);
+        row(get(min(t + 1, nt - 1)).k, kn);
+        __builtin_amdgcn_sched_barrier(0);   // the LDS reads are out before the sum over the row groups
+        const float sum = sum_row_groups(kv);   // (rg 0 + rg 1) + (rg 2 + rg 3), the same bits in all four lanes
+        const float delta = (tk.v - tk.g * sum) * tk.beta;
+        float o = 0.0f, kvn = 0.0f;
+#pragma unroll
+        for (int r = 0; r < RPG; ++r) {
+            s[r] = __builtin_fmaf(tk.g, s[r], k[r] * delta);
+            o = __builtin_fmaf(s[r], q[r], o);
+            kvn = __builtin_fmaf(s[r], kn[r], kvn);
+        }
+        part[64 * t + static_cast<int>(threadIdx.x & 63)] = o;
+        kv = kvn;
+    };
+    // pairs (the k rows change places without register moves), then the odd token
+    int t = 0;
+    for (; t + 1 < nt; t += 2) {
+        step(t, ka, kb);
+        step(t + 1, kb, ka);
+    }
+    if (t < nt) step(t, ka, kb);
+}
+
+// lane l of the wave that wrote part: token l / 4's outputs (scaled) at columns 4 (l % 4) .. + 3 of the 16; with l % 4 = 0
+// the sum of the 16 squares as the butterfly of gdn_step_kernel's lane 0 forms it (the first step's square is contracted
+// into its addition)
+__device__ __forceinline__ float4 scan_outputs(const float* part, int ln, float& squares) {
+    const float* p = part + 64 * (ln >> 2) + 4 * (ln & 3);
+    float oc[4];
+    const float4 r0 = *reinterpret_cast<const float4*>(p), r1 = *reinterpret_cast<const float4*>(p + 16);
+    const float4 r2 = *reinterpret_cast<const float4*>(p + 32), r3 = *reinterpret_cast<const float4*>(p + 48);
+    oc[0] = ((r0.x + r1.x) + (r2.x + r3.x)) * 0.08838834764831845f;   // 1 / sqrt(128)
+    oc[1] = ((r0.y + r1.y) + (r2.y + r3.y)) * 0.08838834764831845f;
+    oc[2] = ((r0.z + r1.z) + (r2.z + r3.z)) * 0.08838834764831845f;
+    oc[3] = ((r0.w + r1.w) + (r2.w + r3.w)) * 0.08838834764831845f;
+    float u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float sq = oc[i] * oc[i];
+        const float t8 = __builtin_fmaf(oc[i], oc[i], xor_lane<2>(sq));   // columns c and c + 8 (lanes l % 4 < 2)
+        u[i] = t8 + xor_lane<1>(t8);                                      // and c + 4
+    }
+    squares = (u[0] + u[2]) + (u[1] + u[3]);
+    return make_float4(oc[0], oc[1], oc[2], oc[3]);
+}
+
+// ---- ingest chunks of 3..16 tokens: four workgroups per value head, then the output norm -----------------------------
+// A chunk's first launch holds each value head's 128 state columns in four parts of 32, as the split kernel does, but
+// leaves the raw outputs in y; the second takes the norm over the head's columns, the gate and the Q8_1 blocks, and
+// writes the conv history, which the first launch's four parts all read.  In a part the four waves share the conv (waves
+// 0, 1 the head's q channels, 2, 3 its k channels, all four the part's v), and waves 0, 1 then run the recurrence on 16
+// columns each.  One workgroup per value head (gdn_step_kernel) had its eight waves queue for the same LDS rows:
+// 16 tokens of the 9B layer 20.9 us; this pair MEASURED.
+constexpr int kChunkTok = kMaxCols;
+
+__global__ __launch_bounds__(2 * S) void gdn_chunk_scan(StepArgs a) {
+    __shared__ __attribute__((aligned(16))) float cqk[2][kChunkTok][S];   // q and k, convolved and normalized
+    __shared__ float cv[kChunkTok][kPartCols];
+    __shared__ float cpart[kChunkTok][4];
+    __shared__ float gbt[kChunkTok][2];
+    __shared__ __attribute__((aligned(16))) float outs[2][kChunkTok * 64];
+    // part-major, as the split kernel: a head's parts on one XCD when h_v is a multiple of 8
+    const int head = static_cast<int>(blockIdx.x) % a.h_v, part = static_cast<int>(blockIdx.x) / a.h_v;
+    const int t = threadIdx.x, wv = t >> 6, ln = t & 63, rg = ln >> 4;
+    const int qh = head % a.h_k, ntok = a.ntok;
+    const int kind = t >> 7, j = t & (S - 1);
+    const int lcol = 16 * (wv & 1) + (ln & 15), col = kPartCols * part + lcol;   // waves 0, 1: state columns
+    const size_t row_stride = static_cast<size_t>(a.h_v) * S;
+    const size_t base = (static_cast<size_t>(rg * RPG) * a.h_v + head) * S + col;
+    const int jv = kPartCols * part + (t & 31), tv = 2 * (t >> 5);   // v: channel jv, tokens tv and tv + 1
+
+    const int selv = a.sel[opaque_zero()];   // first: the state addresses depend on it
+    const float* src = (kind == 0 ? a.q : a.k) + qh * S + j;
+    float x[kChunkTok + 3], xv[5];
+#pragma unroll
+    for (int i = 0; i < kChunkTok; ++i) x[i + 3] = src[static_cast<size_t>(min(i, ntok - 1)) * a.tok_stride];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) xv[i] = a.v[static_cast<size_t>(min(max(tv + i - 3, 0), ntok - 1)) * a.tok_stride + head * S + jv];
+    const int c = (kind * a.h_k + qh) * S + j, cvc = (2 * a.h_k + head) * S + jv;
+    float w[4], wvv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w[i] = a.conv_w[4 * c + i];
+        wvv[i] = a.conv_w[4 * cvc + i];
+    }
+    const int gt = min(t & 63, ntok - 1);   // the gates: wave 3's lane gt
+    const float* ab = a.ab + static_cast<size_t>(gt) * a.ab_stride;
+    const float gin[4] = {ab[head], ab[a.h_v + head], a.dt[head], a.ssm_a[head]};
+    const int ch = (3 * head + kind) * S + j, chv = (3 * head + 2) * S + jv;
+    float h[2][3], hv[2][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        h[0][i] = a.hist_a[3 * ch + i];
+        h[1][i] = a.hist_b[3 * ch + i];
+        hv[0][i] = a.hist_a[3 * chv + i];
+        hv[1][i] = a.hist_b[3 * chv + i];
+    }
+    const bool sel_b = selv != 0;
+    float* state = sel_b ? a.state_b : a.state_a;
+    __builtin_amdgcn_sched_barrier(0);
+    float s[RPG];
+    if (wv < 2) {
+#pragma unroll
+        for (int r = 0; r < RPG; ++r) s[r] = __builtin_nontemporal_load(state + base + r * row_stride);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) x[i] = sel_b ? h[1][i] : h[0][i];
+
+    if (wv == 3 && (t & 63) < ntok) gate_values(gin[0], gin[1], gin[2], gin[3], gbt[gt][0], gbt[gt][1]);
+    float y[kChunkTok];
+#pragma unroll
+    for (int i = 0; i < kChunkTok; ++i) {
+        y[i] = silu(__builtin_fmaf(x[i + 3], w[3], __builtin_fmaf(x[i + 2], w[2], __builtin_fmaf(x[i + 1], w[1], x[i] * w[0]))));
+        const float sqs = group_sum<64>(y[i] * y[i]);
+        if (ln == 0) cpart[i][wv] = sqs;
+    }
+    // v: a token before the first comes from the history
+    if (tv < 3) {   // uniform per half wave
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int b = tv + i;   // entry b of [h0 h1 h2 | x_0 ..]
+            const float hb = b == 0 ? (sel_b ? hv[1][0] : hv[0][0]) : b == 1 ? (sel_b ? hv[1][1] : hv[0][1]) : (sel_b ? hv[1][2] : hv[0][2]);
+            if (b < 3) xv[i] = hb;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        cv[tv + i][t & 31] = silu(__builtin_fmaf(xv[i + 3], wvv[3],
+                                                 __builtin_fmaf(xv[i + 2], wvv[2], __builtin_fmaf(xv[i + 1], wvv[1], xv[i] * wvv[0]))));
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kChunkTok; ++i)
+        cqk[kind][i][j] = y[i] * rsqrtf((cpart[i][2 * kind] + cpart[i][2 * kind + 1]) + a.eps);
+    __syncthreads();
+    if (wv >= 2) return;
+    scan_tokens(s, ntok, rg, outs[wv], [&](int i) {
+        return ScanToken{cqk[0][i], cqk[1][i], gbt[i][0], gbt[i][1], cv[i][lcol]};
+    });
+#pragma unroll
+    for (int r = 0; r < RPG; ++r) __builtin_nontemporal_store(s[r], state + base + r * row_stride);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own part rows
+    float ss;
+    const float4 oc = scan_outputs(outs[wv], ln, ss);
+    const int tt = ln >> 2;
+    if (tt < ntok) {
+        float* o = a.y + static_cast<size_t>(tt) * a.y_stride + head * S + kPartCols * part + 16 * wv + 4 * (ln & 3);
+        o[0] = oc.x;
+        o[1] = oc.y;
+        o[2] = oc.z;
+        o[3] = oc.w;
+    }
+}
+
+// token blockIdx.y of head blockIdx.x: the norm over the head's raw outputs (its eight 16-column sums in order), the gate,
+// y and its Q8_1 blocks; the first token's workgroup also writes the head's conv history (the last three inputs)
+__global__ __launch_bounds__(S) void gdn_chunk_finish(StepArgs a) {
+    __shared__ float wsum[S / 16];
+    const int head = blockIdx.x, t = blockIdx.y, col = threadIdx.x;
+    float* y = a.y + static_cast<size_t>(t) * a.y_stride + head * S + col;
+    const float oc = *y;
+    const float zz = a.z[static_cast<size_t>(t) * a.tok_stride + head * S + col];
+    const float gam = a.gamma[col];
+    const float sq = oc * oc;
+    float u = __builtin_fmaf(oc, oc, xor_lane<8>(sq));   // the order of gdn_step_kernel's 16-column sums, lane 0's result
+    u += xor_lane<4>(u);
+    u += xor_lane<2>(u);
+    u += xor_lane<1>(u);
+    if ((col & 15) == 0) wsum[col >> 4] = u;
+    if (t == 0) {
+        const int qh = head % a.h_k;
+        float* hist = *a.sel != 0 ? a.hist_b : a.hist_a;
+#pragma unroll
+        for (int kind = 0; kind < 3; ++kind) {
+            const float* src = (kind == 0 ? a.q + qh * S : kind == 1 ? a.k + qh * S : a.v + head * S) + col;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                hist[3 * ((3 * head + kind) * S + col) + i] = src[static_cast<size_t>(a.ntok - 3 + i) * a.tok_stride];
+        }
+    }
+    __syncthreads();
+    float tot = 0.0f;
+#pragma unroll
+    for (int w = 0; w < S * RG / 64; ++w) tot += wsum[w];
+    const float scl = rsqrtf(tot / static_cast<float>(S) + a.eps);
+    const float yv = oc * scl * gam * silu(zz);
+    *y = yv;
+    if (a.q8) q8_1_store_lane(yv, a.q8 + static_cast<size_t>(t) * a.q8_stride + (head * 4 + (col >> 5)) * kQ8_1Bytes);
+}
+
 // ---- wide ingest chunks: conv, recurrence and output norm as three launches -------------------------------------------
 // Only the recurrence is serial in the tokens.  (1) gdn_wide_prep runs the conv + SiLU + L2 and the gates of every token
 // in parallel; (2) gdn_wide_scan walks the tokens with one wave per 16 columns of a value head, the state in its
@@ -794,8 +1011,7 @@ __global__ __launch_bounds__(64) void gdn_wide_scan(WideArgs w) {
     __shared__ __attribute__((aligned(16))) float sqk[2][kScanTok][2 * S];
     __shared__ __attribute__((aligned(16))) float sv[2][kScanTok][16];
     __shared__ __attribute__((aligned(16))) float sgb[2][2 * kScanTok][2];
-    __shared__ __attribute__((aligned(16))) float so[kScanTok][16];
-    __shared__ float sw[kScanTok];
+    __shared__ __attribute__((aligned(16))) float part[kScanTok * 64];
     // workgroup w * h_v + head: round robin over the XCDs, so a head's eight waves (h_v a multiple of 8) share an L2
     const int head = static_cast<int>(blockIdx.x) % a.h_v, wv = static_cast<int>(blockIdx.x) / a.h_v;
     const int ln = threadIdx.x, rg = ln >> 4;
@@ -831,47 +1047,17 @@ __global__ __launch_bounds__(64) void gdn_wide_scan(WideArgs w) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         const int nt = min(kScanTok, a.ntok - t0);
         if (t0 + kScanTok < a.ntok) fetch(t0 + kScanTok, b ^ 1);
-        float k[RPG], kv = 0.0f;
-#pragma unroll
-        for (int r4 = 0; r4 < RPG / 4; ++r4)
-            *reinterpret_cast<float4*>(k + 4 * r4) = *reinterpret_cast<const float4*>(&sqk[b][0][S + rg * RPG + 4 * r4]);
-#pragma unroll
-        for (int r = 0; r < RPG; ++r) kv = __builtin_fmaf(s[r], k[r], kv);
-        for (int t = 0; t < nt; ++t) {
-            float q[RPG], kn[RPG];
-            const int tn = min(t + 1, kScanTok - 1);
-#pragma unroll
-            for (int r4 = 0; r4 < RPG / 4; ++r4) {
-                *reinterpret_cast<float4*>(q + 4 * r4) = *reinterpret_cast<const float4*>(&sqk[b][t][rg * RPG + 4 * r4]);
-                *reinterpret_cast<float4*>(kn + 4 * r4) =
-                    *reinterpret_cast<const float4*>(&sqk[b][tn][S + rg * RPG + 4 * r4]);
-            }
-            const float g = sgb[b][t][0], beta = sgb[b][t][1];
-            const float vcol = sv[b][t][ln & 15];
-            kv = sum_row_groups(kv);
-            const float delta = (vcol - g * kv) * beta;
-            float o = 0.0f, kvn = 0.0f;
-#pragma unroll
-            for (int r = 0; r < RPG; ++r) {
-                s[r] = __builtin_fmaf(g, s[r], k[r] * delta);
-                o = __builtin_fmaf(s[r], q[r], o);
-                kvn = __builtin_fmaf(s[r], kn[r], kvn);
-            }
-            o = sum_row_groups(o);
-            const float oc = o * 0.08838834764831845f;   // 1 / sqrt(128)
-            const float ss = group_sum<16>(oc * oc);
-            if (rg == 0) so[t][ln] = oc;
-            if (ln == 0) sw[t] = ss;
-            kv = kvn;
-#pragma unroll
-            for (int r = 0; r < RPG; ++r) k[r] = kn[r];
-        }
+        scan_tokens(s, nt, rg, part, [&](int t) {
+            return ScanToken{sqk[b][t], sqk[b][t] + S, sgb[b][t][0], sgb[b][t][1], sv[b][t][ln & 15]};
+        });
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        float ss;
+        const float4 oc = scan_outputs(part, ln, ss);
         const int tt = ln >> 2;
-        if (tt < nt)
-            *reinterpret_cast<float4*>(a.y + static_cast<size_t>(t0 + tt) * a.y_stride + head * S + 16 * wv + 4 * (ln & 3)) =
-                *reinterpret_cast<const float4*>(&so[tt][4 * (ln & 3)]);
-        if (ln < nt) w.wsum[(static_cast<size_t>(t0 + ln) * a.h_v + head) * 8 + wv] = sw[ln];
+        if (tt < nt) {
+            *reinterpret_cast<float4*>(a.y + static_cast<size_t>(t0 + tt) * a.y_stride + head * S + 16 * wv + 4 * (ln & 3)) = oc;
+            if ((ln & 3) == 0) w.wsum[(static_cast<size_t>(t0 + tt) * a.h_v + head) * 8 + wv] = ss;
+        }
     }
 #pragma unroll
     for (int r = 0; r < RPG; ++r) state[base + r * row_stride] = s[r];
@@ -1004,7 +1190,8 @@ int gdn_layer(float* state_a, float* state_b, float* hist_a, float* hist_b, cons
     } else if (ntok == 1) {
         hipLaunchKernelGGL((gdn_step_kernel<1, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
     } else {
-        hipLaunchKernelGGL((gdn_step_kernel<kMaxCols, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
+        hipLaunchKernelGGL(gdn_chunk_scan, dim3(h_v * kParts), dim3(2 * S), 0, s, a);
+        hipLaunchKernelGGL(gdn_chunk_finish, dim3(h_v, ntok), dim3(S), 0, s, a);
     }
     return launch_status("gdn_layer_tokens");
 }
