@@ -126,9 +126,12 @@ constexpr int KTILE = STEP * KROW;       // 8448 bytes per wave; reused for the 
 __device__ __forceinline__ void lds_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
-// K / V rows are streamed once per step: nontemporal loads, as the GEMVs stream their weights
+// K / V rows: one slot group streams each once (nontemporal loads, as the GEMVs stream their weights); several groups
+// read the same rows, which the first then leaves in the L2 (SHARED)
+template <bool SHARED>
 __device__ __forceinline__ uint4 load_kv(const uint16_t* p) {
-    const u32x4v v = __builtin_nontemporal_load(reinterpret_cast<const u32x4v*>(p));
+    const auto* q = reinterpret_cast<const u32x4v*>(p);
+    const u32x4v v = SHARED ? *q : __builtin_nontemporal_load(q);
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
@@ -172,21 +175,32 @@ struct PrepIn {
 };
 constexpr int kRopeOwn = 0, kRopeWrite = 1, kRopeRead = 2;
 
-template <bool PREP>
+// SHARED (several slot groups): a one-dimensional grid of groups x (chunk, KV head) pairs, padded to a multiple of 8
+// pairs, in which the groups of a pair are consecutive workgroups of one XCD (workgroups go to the XCDs round robin), so
+// its K / V rows come from HBM once.  Group-major order with nontemporal loads fetched them once per group: this launch
+// 29.6 us at 16 tokens behind 4K positions (1024 workgroups of two steps), this order 26.1 us; the whole call 33.7 ->
+// 31.2 us.  What is left is each workgroup's own chain (position, query rows, first K / V rows, two steps, combine).
+template <bool PREP, bool SHARED>
 __global__ __launch_bounds__(256, 2) void gqa_partial_kernel(const float* __restrict__ qbuf, const uint16_t* __restrict__ kc,
                                                           const uint16_t* __restrict__ vc, const int* __restrict__ pos,
                                                           float* __restrict__ ws, int slot_stride, int n_head,
                                                           int n_kv, int ntok, int nsub, int max_ctx, float scale,
-                                                          PrepIn pr) {
+                                                          int npairs, PrepIn pr) {
     __shared__ __attribute__((aligned(16))) uint8_t tiles[WAVES * KTILE];
     __shared__ float wstat[WAVES][2][SLOTS];
     __shared__ float pred[PREP ? 2 : 1][WAVES];   // PREP: wave sums of the new K rows
     // the KV heads of one chunk are neighbouring workgroups (dispatched together), so the four 512-byte head rows of a
     // position are read close in time
-    const int chunk = static_cast<int>(blockIdx.x) / n_kv, kv = static_cast<int>(blockIdx.x) - chunk * n_kv;
-    const int s0 = SLOTS * static_cast<int>(blockIdx.z);
     const int G = n_head / n_kv;
     const int nq = ntok * G;
+    int pair = static_cast<int>(blockIdx.x), s0 = 0;
+    if constexpr (SHARED) {
+        const int groups = (nq + SLOTS - 1) / SLOTS, i = pair >> 3, k = i / groups;
+        s0 = SLOTS * (i - k * groups);
+        pair = 8 * k + (pair & 7);
+        if (pair >= npairs) return;
+    }
+    const int chunk = pair / n_kv, kv = pair - chunk * n_kv;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int l16 = lane & 15, g4 = lane >> 4;
     const int slot = s0 + (l16 & 7);   // query slot t * G + gh of this lane's MFMA column / row
@@ -327,15 +341,15 @@ __global__ __launch_bounds__(256, 2) void gqa_partial_kernel(const float* __rest
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int p = min(wbase + 2 * j + krow, wlast);
-        set_u4(kreg, j, load_kv(kb + p * rstride + kcol * 8));
+        set_u4(kreg, j, load_kv<SHARED>(kb + p * rstride + kcol * 8));
     }
     // V of a step: [2 j + dg] = position sb + 4 g4 + j, dims 128 dg + 8 l16 + [0, 8); also one step ahead
     u32x32 vnext;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint16_t* vr = vb + min(wbase + 4 * g4 + j, wlast) * rstride + 8 * l16;
-        set_u4(vnext, 2 * j, load_kv(vr));
-        set_u4(vnext, 2 * j + 1, load_kv(vr + 128));
+        set_u4(vnext, 2 * j, load_kv<SHARED>(vr));
+        set_u4(vnext, 2 * j + 1, load_kv<SHARED>(vr + 128));
     }
     // the new rows' inputs and the table's K entries stay live until the K / V loads are out: reusing their registers
     // for the K / V addresses made those loads wait for every load of the prologue
@@ -404,8 +418,8 @@ __global__ __launch_bounds__(256, 2) void gqa_partial_kernel(const float* __rest
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint16_t* vr = vb + min(sb + STEP + 4 * g4 + j, wlast) * rstride + 8 * l16;
-            set_u4(vnext, 2 * j, load_kv(vr));
-            set_u4(vnext, 2 * j + 1, load_kv(vr + 128));
+            set_u4(vnext, 2 * j, load_kv<SHARED>(vr));
+            set_u4(vnext, 2 * j + 1, load_kv<SHARED>(vr + 128));
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) *reinterpret_cast<uint4*>(kt + (2 * j + krow) * KROW + kcol * 16) = get_u4(kreg, j);
@@ -413,7 +427,7 @@ __global__ __launch_bounds__(256, 2) void gqa_partial_kernel(const float* __rest
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int p = min(sb + STEP + 2 * j + krow, wlast);
-            set_u4(kreg, j, load_kv(kb + p * rstride + kcol * 8));
+            set_u4(kreg, j, load_kv<SHARED>(kb + p * rstride + kcol * 8));
         }
         lds_wave_sync();
         floatx4 sacc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -687,8 +701,13 @@ int flash_decode(const float* q, const uint16_t* kcache, const uint16_t* vcache,
                  int gate_stride, float* y, int y_stride, uint8_t* q8, int q8_stride, float* ws, int slot_stride,
                  int n_head, int n_kv, int ntok, int nchunks, int nsub, int max_ctx, float scale, hipStream_t s) {
     const int groups = (ntok * (n_head / n_kv) + SLOTS - 1) / SLOTS;
-    hipLaunchKernelGGL(gqa_partial_kernel<false>, dim3(nchunks * n_kv, 1, groups), dim3(256), 0, s, q, kcache, vcache, pos,
-                       ws, slot_stride, n_head, n_kv, ntok, nsub, max_ctx, scale, PrepIn{});
+    const int npairs = nchunks * n_kv;
+    if (groups > 1)
+        hipLaunchKernelGGL((gqa_partial_kernel<false, true>), dim3((npairs + 7) / 8 * 8 * groups), dim3(256), 0, s, q, kcache,
+                           vcache, pos, ws, slot_stride, n_head, n_kv, ntok, nsub, max_ctx, scale, npairs, PrepIn{});
+    else
+        hipLaunchKernelGGL((gqa_partial_kernel<false, false>), dim3(npairs), dim3(256), 0, s, q, kcache, vcache, pos, ws,
+                           slot_stride, n_head, n_kv, ntok, nsub, max_ctx, scale, npairs, PrepIn{});
     hipLaunchKernelGGL(gqa_merge_kernel, dim3(ntok, n_head, kMergeParts), dim3(HD), 0, s, ws, slot_stride, gate_src, gate_stride,
                        pos, y, y_stride, q8, q8_stride, n_head, n_kv, SUB * nsub);
     return launch_status("gqa_flash_decode");
@@ -812,8 +831,8 @@ int flash_decode_prep(const float* q3, int q3_stride, const float* qn, const flo
                     reinterpret_cast<float2*>(rope_cs), cs_mode};
     const auto s = static_cast<hipStream_t>(stream);
     auto* ws = static_cast<float*>(workspace);
-    hipLaunchKernelGGL(gqa_partial_kernel<true>, dim3(nchunks * n_kv, 1, 1), dim3(256), 0, s, nullptr, kcache, vcache,
-                       pos, ws, kMaxSlots, n_head, n_kv, ntok, nsub, max_ctx, scale, pr);
+    hipLaunchKernelGGL((gqa_partial_kernel<true, false>), dim3(nchunks * n_kv, 1, 1), dim3(256), 0, s, nullptr, kcache,
+                       vcache, pos, ws, kMaxSlots, n_head, n_kv, ntok, nsub, max_ctx, scale, nchunks * n_kv, pr);
     hipLaunchKernelGGL(gqa_merge_kernel, dim3(ntok, n_head, kMergeParts), dim3(HD), 0, s, ws, kMaxSlots, q3, q3_stride,
                        pos, y, y_stride, q8, q8_stride, n_head, n_kv, SUB * nsub);
     return launch_status("gqa_flash_decode_prep");
