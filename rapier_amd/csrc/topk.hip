@@ -5,12 +5,16 @@
 // then the inverted id), all keys are distinct, and the list is the k largest keys in descending order: the same
 // (logit descending, id ascending) order.
 //
-// Two launches.  topk_lists: one wave per 64*E consecutive logits; each lane sorts its E keys in registers (a bitonic
-// network, compile-time indices), then k rounds of a wave max over the lanes' heads pop the wave's k largest into a
-// sorted list (one key per lane, 0 past k); the four waves of a workgroup then merge their lists into one.
-// topk_merge: one 512-lane workgroup merges the workgroups' lists pairwise, level by level, in LDS.  Two sorted lists
-// merge in one wave: lane l takes max(A[l], B[63 - l]), the top half of the bitonic sequence A | reverse(B), i.e. the
-// 64 largest keys of both, and a bitonic half-cleaner network (lane strides 32 .. 1) sorts them.
+// Two launches of bitonic networks whose lanes hold the keys (compile-time lane strides, VALU exchanges).  topk_lists: a
+// wave takes 256 consecutive logits at a time, four keys per lane, sorts each of the four 64-key registers across its
+// lanes (21 exchanges, the four independent of one another), and merges them and its list so far into the 64 largest;
+// the eight waves of a workgroup then merge theirs.  topk_merge: one workgroup of 16 waves; each loads eight workgroup
+// lists and merges them in registers, and the 16 results meet in LDS four to a wave.  Two sorted lists merge in one
+// wave: lane l takes max(A[l], B[63 - l]), the top half of the bitonic sequence A | reverse(B), i.e. the 64 largest keys
+// of both, and a bitonic half-cleaner network (lane strides 32 .. 1) sorts them; B is kept ascending, so no lane
+// reversal is needed.
+// Both are bound by their chains of exchanges.  Popping the k largest by k wave-wide maxima (13.3 us at 248320 logits
+// and k = 40) and merging the lists pair by pair through LDS (12.4 us) took 1.6x as long: 8.6 and 7.3 us here.
 #include "rmi_common.h"
 
 namespace rmi {
@@ -18,43 +22,15 @@ namespace {
 
 constexpr int kTopkMax = 64;       // largest k
 constexpr int kListStride = 64;    // keys per list in the workspace
-constexpr int kMergeLanes = 512;   // waves of the list pass at most (4 per workgroup list)
-constexpr int kMaxLists = kMergeLanes / 4;   // workgroup lists the merge holds in LDS (64 KB)
+constexpr int kListWaves = 8;      // waves of a list workgroup
+constexpr int kMaxLists = 128;     // workgroup lists the merge takes: 8 per wave
+constexpr int kMergeWaves = 16;
 
 __device__ __forceinline__ uint64_t topk_key(float v, uint32_t idx) {
     uint32_t b = __float_as_uint(v);
     if (b == 0x80000000u) b = 0u;   // -0 compares equal to +0
     b ^= (b >> 31) ? 0xffffffffu : 0x80000000u;
     return (static_cast<uint64_t>(b) << 32) | (0xffffffffu - idx);   // > 0 for every real key; 0 = no entry
-}
-
-__device__ __forceinline__ uint64_t max64(uint64_t a, uint64_t b) { return a > b ? a : b; }
-
-// lane exchange by a DPP pattern (every lane active)
-template <int CTRL>
-__device__ __forceinline__ uint64_t dpp64(uint64_t v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<uint32_t>(v)), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<uint32_t>(v >> 32)), CTRL, 0xf, 0xf,
-                                               false);
-    return (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo);
-}
-
-__device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), lane));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v >> 32)),
-                                                                        lane));
-    return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
-// wave-uniform max of a 64-bit key: DPP within each row of 16 lanes (xor 1, xor 2, half-row mirror, row mirror; max
-// is symmetric, so a mirror partner serves as well as an xor one), then the four row maxima read into scalars.
-// Called with every lane of the wave active.
-__device__ __forceinline__ uint64_t wave_max64(uint64_t k) {
-    k = max64(k, dpp64<0xb1>(k));    // quad_perm [1,0,3,2]
-    k = max64(k, dpp64<0x4e>(k));    // quad_perm [2,3,0,1]
-    k = max64(k, dpp64<0x141>(k));   // row_half_mirror
-    k = max64(k, dpp64<0x140>(k));   // row_mirror
-    return max64(max64(readlane64(k, 0), readlane64(k, 16)), max64(readlane64(k, 32), readlane64(k, 48)));
 }
 
 // key of lane l ^ K (the VALU lane exchange of rmi_common.h on both halves)
@@ -64,136 +40,133 @@ __device__ __forceinline__ uint64_t xor64(uint64_t v) {
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+// one compare-exchange with lane l ^ K: the larger key where `larger` holds (equal keys are the same key, or both 0)
 template <int K>
-__device__ __forceinline__ uint64_t half_clean(uint64_t v, int lane) {
+__device__ __forceinline__ uint64_t exchange(uint64_t v, bool larger) {
     const uint64_t o = xor64<K>(v);
-    return (lane & K) ? (v < o ? v : o) : (v > o ? v : o);
+    return (v > o) == larger ? v : o;
 }
 
-// The 64 largest keys of two descending lists, descending, one per lane: a = A[lane], b = B[63 - lane].  Called with
-// every lane of the wave active.
-__device__ __forceinline__ uint64_t merge_lists(uint64_t a, uint64_t b) {
-    const int lane = __lane_id();
-    uint64_t v = a > b ? a : b;
-    v = half_clean<32>(v, lane);
-    v = half_clean<16>(v, lane);
-    v = half_clean<8>(v, lane);
-    v = half_clean<4>(v, lane);
-    v = half_clean<2>(v, lane);
-    return half_clean<1>(v, lane);
+// the bitonic network's last stage: a bitonic sequence over the wave's lanes into descending (ASC: ascending) order
+template <bool ASC, int K = 32>
+__device__ __forceinline__ uint64_t half_clean(uint64_t v, int lane) {
+    v = exchange<K>(v, ((lane & K) == 0) != ASC);
+    if constexpr (K > 1) v = half_clean<ASC, K / 2>(v, lane);
+    return v;
 }
 
-template <int E>
-__global__ __launch_bounds__(256) void topk_lists_kernel(const float* __restrict__ x, int n, int k,
-                                                         uint64_t* __restrict__ lists) {
-    const int lane = threadIdx.x & 63;
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t base = static_cast<int64_t>(wave) * 64 * E;
-    // every load issued before the first use, from clamped indices (a load under a branch gets a wait of its own)
-    float xv[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) xv[j] = x[min(base + lane + 64 * j, static_cast<int64_t>(n) - 1)];
-    uint64_t v[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-        const int64_t i = base + lane + 64 * j;
-        v[j] = i < n ? topk_key(xv[j], static_cast<uint32_t>(i)) : 0ull;
-    }
-    // bitonic sort of the lane's E keys, descending
-#pragma unroll
-    for (int size = 2; size <= E; size <<= 1) {
-#pragma unroll
-        for (int stride = size / 2; stride > 0; stride >>= 1) {
-#pragma unroll
-            for (int i = 0; i < E; ++i) {
-                const int j = i ^ stride;
-                if (j > i) {
-                    const uint64_t a = v[i], b = v[j];
-                    const bool swap = (i & size) == 0 ? a < b : a > b;
-                    v[i] = swap ? b : a;
-                    v[j] = swap ? a : b;
-                }
-            }
-        }
-    }
-    uint64_t mine = 0;
-    for (int it = 0; it < k; ++it) {
-        const uint64_t m = wave_max64(v[0]);
-        if (m == 0) break;              // the slice has fewer than k logits (uniform across the wave)
-        if (lane == it) mine = m;
-        if (v[0] == m) {                // keys are distinct: exactly one lane pops
-#pragma unroll
-            for (int j = 0; j + 1 < E; ++j) v[j] = v[j + 1];
-            v[E - 1] = 0;
-        }
-    }
-    // the workgroup's four lists into one: waves 0 / 1 merge lists (0, 1) / (2, 3), then wave 0 merges the two
-    __shared__ uint64_t wl[4][64];
-    const int w = threadIdx.x >> 6;
-    wl[w][lane] = mine;
-    __syncthreads();
-    uint64_t m2 = 0;
-    if (w < 2) m2 = merge_lists(wl[2 * w][lane], wl[2 * w + 1][63 - lane]);
-    __syncthreads();
-    if (w < 2) wl[w][lane] = m2;
-    __syncthreads();
-    if (w == 0) lists[static_cast<size_t>(blockIdx.x) * kListStride + lane] = merge_lists(wl[0][lane], wl[1][63 - lane]);
+// The 64 largest keys of a (descending) and b (ascending), in descending (ASC: ascending) order.  Every lane active.
+template <bool ASC>
+__device__ __forceinline__ uint64_t merge_lists(uint64_t a, uint64_t b, int lane) {
+    return half_clean<ASC>(a > b ? a : b, lane);
 }
 
-// Workgroup lists merged pairwise: each level reads every pair into registers (wave w takes pairs w, w + 8, ...), passes
-// a barrier, and writes the merged lists to the first half of the slots; an odd last list moves down with them.
-__global__ __launch_bounds__(kMergeLanes) void topk_merge_kernel(const float* __restrict__ x,
-                                                                 const uint64_t* __restrict__ lists, int nlists, int k,
-                                                                 int* __restrict__ out_idx, float* __restrict__ out_val) {
-    __shared__ uint64_t buf[kMaxLists * kListStride];
-    constexpr int kWaves = kMergeLanes / 64;
-    constexpr int kPer = kMaxLists / 2 / kWaves;   // pairs per wave at the widest level
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    {   // every list entry of the lane loaded before the first store (a strided loop waits on each load in turn)
-        constexpr int kLoads = kMaxLists * kListStride / kMergeLanes;
-        const int total = nlists * kListStride;
-        uint64_t lv[kLoads];
+// one stage of the sort: runs of SIZE lanes, alternately descending and ascending (ASC: the other way round)
+template <bool ASC, int SIZE, int K = SIZE / 2>
+__device__ __forceinline__ uint64_t sort_stage(uint64_t v, int lane) {
+    v = exchange<K>(v, (((lane & K) == 0) != ((lane & SIZE) != 0)) != ASC);
+    if constexpr (K > 1) v = sort_stage<ASC, SIZE, K / 2>(v, lane);
+    return v;
+}
+template <bool ASC>
+__device__ __forceinline__ uint64_t sort64(uint64_t v, int lane) {
+    v = sort_stage<ASC, 2>(v, lane);
+    v = sort_stage<ASC, 4>(v, lane);
+    v = sort_stage<ASC, 8>(v, lane);
+    v = sort_stage<ASC, 16>(v, lane);
+    v = sort_stage<ASC, 32>(v, lane);
+    return sort_stage<ASC, 64>(v, lane);   // lane & 64 is 0
+}
+
+// `groups` slices of 256 logits per wave
+__global__ __launch_bounds__(64 * kListWaves) void topk_lists_kernel(const float* __restrict__ x, int n, int groups,
+                                                                     uint64_t* __restrict__ lists) {
+    __shared__ uint64_t wl[kListWaves][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t base = (static_cast<int64_t>(blockIdx.x) * kListWaves + w) * groups * 256 + lane;
+    const int64_t last = n - 1;
+    float xv[4];
 #pragma unroll
-        for (int r = 0; r < kLoads; ++r) lv[r] = lists[min(t + kMergeLanes * r, total - 1)];
+    for (int j = 0; j < 4; ++j) xv[j] = x[min(base + 64 * j, last)];   // clamped: no load under a branch
+    uint64_t mine = 0;   // the wave's list, descending
+    for (int g = 0; g < groups; ++g) {
+        const int64_t i0 = base + 256 * g;
+        uint64_t v[4];
 #pragma unroll
-        for (int r = 0; r < kLoads; ++r)
-            if (t + kMergeLanes * r < total) buf[t + kMergeLanes * r] = lv[r];
+        for (int j = 0; j < 4; ++j) {
+            const int64_t i = i0 + 64 * j;
+            v[j] = i < n ? topk_key(xv[j], static_cast<uint32_t>(i)) : 0ull;
+            xv[j] = x[min(i + 256, last)];   // the next slice's, in flight during this one's sort
+        }
+        v[0] = sort64<false>(v[0], lane);
+        v[1] = sort64<true>(v[1], lane);
+        v[2] = sort64<false>(v[2], lane);
+        v[3] = sort64<true>(v[3], lane);
+        const uint64_t a = merge_lists<false>(v[0], v[1], lane), b = merge_lists<true>(v[2], v[3], lane);
+        if (g == 0) {
+            mine = merge_lists<false>(a, b, lane);
+        } else {
+            mine = merge_lists<false>(mine, merge_lists<true>(a, b, lane), lane);
+        }
+    }
+    // the workgroup's lists: odd waves' ascending
+    wl[w][w & 1 ? 63 - lane : lane] = mine;
+    __syncthreads();
+    uint64_t m = 0;
+    if (w < 2) {
+        const uint64_t a = merge_lists<false>(wl[4 * w][lane], wl[4 * w + 1][lane], lane);
+        m = merge_lists<false>(a, merge_lists<true>(wl[4 * w + 2][lane], wl[4 * w + 3][lane], lane), lane);
     }
     __syncthreads();
-    for (int n = nlists; n > 1;) {
-        const int pairs = n >> 1;
-        uint64_t res[kPer], last = 0;
+    if (w == 1) wl[1][63 - lane] = m;
+    __syncthreads();
+    if (w == 0) lists[static_cast<size_t>(blockIdx.x) * kListStride + lane] = merge_lists<false>(m, wl[1][lane], lane);
+}
+
+__global__ __launch_bounds__(64 * kMergeWaves) void topk_merge_kernel(const float* __restrict__ x,
+                                                                      const uint64_t* __restrict__ lists, int nlists, int k,
+                                                                      int* __restrict__ out_idx,
+                                                                      float* __restrict__ out_val) {
+    __shared__ uint64_t buf[kMergeWaves][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint64_t v[8];   // lists 8 w + j: odd ones read backwards, so ascending
 #pragma unroll
-        for (int r = 0; r < kPer; ++r) {
-            const int p = w + kWaves * r;
-            res[r] = p < pairs ? merge_lists(buf[(2 * p) * kListStride + lane], buf[(2 * p + 1) * kListStride + 63 - lane])
-                               : 0;
-        }
-        if ((n & 1) && w == 0) last = buf[(n - 1) * kListStride + lane];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kPer; ++r) {
-            const int p = w + kWaves * r;
-            if (p < pairs) buf[p * kListStride + lane] = res[r];
-        }
-        if ((n & 1) && w == 0) buf[pairs * kListStride + lane] = last;
-        __syncthreads();
-        n = pairs + (n & 1);
+    for (int j = 0; j < 8; ++j) {
+        const int l = 8 * w + j;
+        const uint64_t e = lists[static_cast<size_t>(min(l, nlists - 1)) * kListStride + (j & 1 ? 63 - lane : lane)];
+        v[j] = l < nlists ? e : 0ull;
     }
-    if (t < k) {
-        const uint64_t key = buf[t];
-        const int idx = key ? static_cast<int>(0xffffffffu - static_cast<uint32_t>(key)) : -1;
-        out_idx[t] = idx;
-        out_val[t] = idx >= 0 ? x[idx] : 0.0f;
+    uint64_t m = 0;
+    if (8 * w < nlists) {   // uniform
+        const uint64_t a = merge_lists<false>(v[0], v[1], lane), b = merge_lists<true>(v[2], v[3], lane);
+        const uint64_t c = merge_lists<false>(v[4], v[5], lane), d = merge_lists<true>(v[6], v[7], lane);
+        m = merge_lists<false>(merge_lists<false>(a, b, lane), merge_lists<true>(c, d, lane), lane);
+    }
+    buf[w][w & 1 ? 63 - lane : lane] = m;
+    __syncthreads();
+    if (w < 4) {
+        const uint64_t a = merge_lists<false>(buf[4 * w][lane], buf[4 * w + 1][lane], lane);
+        m = merge_lists<false>(a, merge_lists<true>(buf[4 * w + 2][lane], buf[4 * w + 3][lane], lane), lane);
+    }
+    __syncthreads();
+    if (w < 4) buf[w][w & 1 ? 63 - lane : lane] = m;
+    __syncthreads();
+    if (w == 0) {
+        const uint64_t a = merge_lists<false>(buf[0][lane], buf[1][lane], lane);
+        m = merge_lists<false>(a, merge_lists<true>(buf[2][lane], buf[3][lane], lane), lane);
+        if (lane < k) {
+            const int idx = m ? static_cast<int>(0xffffffffu - static_cast<uint32_t>(m)) : -1;
+            out_idx[lane] = idx;
+            out_val[lane] = idx >= 0 ? x[idx] : 0.0f;
+        }
     }
 }
 
-// logits per lane of the list pass: the smallest of 8, 16, 32 that keeps the lists within one merge workgroup
+// logits per lane of four list waves (a workgroup's logits / 256): the smallest of 8, 16, 32 that keeps the lists within
+// one merge workgroup
 int lane_elems(int n) {
-    for (int e = 8; e <= 32; e *= 2) {
-        const int64_t waves = (static_cast<int64_t>(n) + 64 * e - 1) / (64 * e);
-        if ((waves + 3) / 4 * 4 <= kMergeLanes) return e;
-    }
+    for (int e = 8; e <= 32; e *= 2)
+        if ((static_cast<int64_t>(n) + 256 * e - 1) / (256 * e) <= kMaxLists) return e;
     return 0;
 }
 
@@ -217,15 +190,12 @@ extern "C" int rmi_topk(const float* logits, int n, int k, int* out_idx, float* 
     if (!aligned4(logits) || !aligned4(out_idx) || !aligned4(out_val) || !workspace ||
         (reinterpret_cast<uintptr_t>(workspace) & 7u) != 0)
         return fail(RMI_ERR_POINTER, "topk: null or misaligned pointer");
-    const int64_t waves = (static_cast<int64_t>(n) + 64 * e - 1) / (64 * e);
-    const int blocks = static_cast<int>((waves + 3) / 4);
+    const int blocks = static_cast<int>((static_cast<int64_t>(n) + 256 * e - 1) / (256 * e));
     auto* lists = static_cast<uint64_t*>(workspace);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (e == 8) hipLaunchKernelGGL(topk_lists_kernel<8>, dim3(blocks), dim3(256), 0, s, logits, n, k, lists);
-    else if (e == 16) hipLaunchKernelGGL(topk_lists_kernel<16>, dim3(blocks), dim3(256), 0, s, logits, n, k, lists);
-    else hipLaunchKernelGGL(topk_lists_kernel<32>, dim3(blocks), dim3(256), 0, s, logits, n, k, lists);
+    hipLaunchKernelGGL(topk_lists_kernel, dim3(blocks), dim3(64 * kListWaves), 0, s, logits, n, e / 8, lists);
     const int rc = launch_status("topk_lists");
     if (rc != RMI_OK) return rc;
-    hipLaunchKernelGGL(topk_merge_kernel, dim3(1), dim3(kMergeLanes), 0, s, logits, lists, blocks, k, out_idx, out_val);
+    hipLaunchKernelGGL(topk_merge_kernel, dim3(1), dim3(64 * kMergeWaves), 0, s, logits, lists, blocks, k, out_idx, out_val);
     return launch_status("topk_merge");
 }
