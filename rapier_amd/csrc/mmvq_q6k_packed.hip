@@ -852,7 +852,7 @@ __global__ __launch_bounds__(64 * NW) void q6k_packed_swiglu(const uint8_t* __re
     }
 }
 
-// ---- ingest GEMM: 8 / 16 columns on the 16-block 4x4x4 int8 MFMA -------------------------------------------------
+// ---- ingest GEMM: up to 8 / 16 columns on the 16-block 4x4x4 int8 MFMA -------------------------------------------------
 // Same wave tiles, lane ownership and fp32 arithmetic as q6k_packed_gemv, with the integer dot products on the matrix
 // cores.  MFMA block b = half-block hb (lanes 4 hb .. 4 hb + 3), A row i = quad row i (the lane's own unpacked
 // weights), B column j = activation column 4 cg + j, and D[i][j] lands in lane 4 hb + j, register i (layout of
@@ -907,7 +907,7 @@ template <int NCG, bool RES, int D, int CS = 1, int KP = 1, int NCHK = 0, bool L
 __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t* __restrict__ wp,
                                                                    const uint8_t* __restrict__ x, float* y,
                                                                    const float* res, float* partials, int n_in,
-                                                                   int n_out) {
+                                                                   int n_out, int ncols) {
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     static_assert(CS == 1 || CS == 2, "column split: one or two waves per quad");
     static_assert(KP == 1 || (KP == 2 && CS == 2 && NCHK % 2 == 0 && NCHK > 0), "two K halves: a wave pair per quad");
@@ -938,7 +938,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
     for (int m = 0; m < kStageRegs; ++m) {
         const int J = min(t + 64 * kWideWaves * m, nb_stage - 1);
         const int col = J / nbs_stage, jb = J - col * nbs_stage;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(col * nbt + jb) * kQ8_1Bytes);
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + jb) * kQ8_1Bytes);
 #pragma unroll
         for (int i = 0; i < 9; ++i) sv[m][i] = p[i];
     }
@@ -972,7 +972,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
     }
     for (int J = t + 64 * kWideWaves * kStageRegs; J < nb_stage; J += 64 * kWideWaves) {
         const int col = J / nbs_stage, jb = J - col * nbs_stage;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(col * nbt + jb) * kQ8_1Bytes);
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + jb) * kQ8_1Bytes);
         uint32_t wv[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) wv[i] = p[i];
@@ -988,7 +988,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
             const int J = min(t + 64 * kWideWaves * m, nb - 1);
             const int col = J / nbs, jb = J - col * nbs;
             const uint32_t* p =
-                reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(col * nbt + nbs + jb) * kQ8_1Bytes);
+                reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + nbs + jb) * kQ8_1Bytes);
 #pragma unroll
             for (int i = 0; i < 9; ++i) pb[m][i] = p[i];
         }
@@ -1111,9 +1111,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
                     }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 // lane o: row io = o / R, group go = (o / 4) % NCW, column jo = o % 4 (lanes past 16 NCW idle)
-                const bool live = lane < 4 * R;
-                const int oo = live ? lane : 0;
+                const int oo = lane < 4 * R ? lane : 0;
                 const int io = oo / R, go = (oo >> 2) % NCW, jo = oo & 3;
+                const bool live = lane < 4 * R && 4 * (NCW * half + go) + jo < ncols;
                 float hv[16];
 #pragma unroll
                 for (int h = 0; h < 16; ++h) hv[h] = lescr[(4 * h + jo) * R + io * NCW + go];
@@ -1157,12 +1157,12 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
                         tot[i][g] = 0.0f;
                         const int row = kQuad * q + i;
                         if constexpr (RES) {
-                            if (row < n_out) v[i] += res[static_cast<size_t>(col) * n_out + row];
+                            if (row < n_out && col < ncols) v[i] += res[static_cast<size_t>(col) * n_out + row];
                         }
-                        if (hb == 0 && row < n_out) y[static_cast<size_t>(col) * n_out + row] = v[i];
+                        if (hb == 0 && row < n_out && col < ncols) y[static_cast<size_t>(col) * n_out + row] = v[i];
                     }
                     if constexpr (RES) {
-                        if (hb == 0) {   // squares of the quad's rows in row order
+                        if (hb == 0 && col < ncols) {   // squares of the quad's rows in row order
                             const int row0 = kQuad * q;
                             float p = __builtin_fmaf(v[0], v[0], 0.0f);
                             if (row0 + 1 < n_out) p = __builtin_fmaf(v[1], v[1], p);
@@ -1312,14 +1312,24 @@ bool wide_halves(int n_in, int n_out) {
            16 * (n_in / 64) <= 64 * kWideWaves * kPhaseRegs && nq <= cu_count() * (kWideWaves / 2);
 }
 
-// the widest ingest pass (16 or 8 columns) whose stage fits kWideStageBytes (16 also in two K halves), or 0
+// columns per narrow pass: at most 4, and the pass's staged activations within kMaxStageBytes
+int cols_per_pass(int n_in) {
+    const int per = kMaxStageBytes / ((n_in / 32) * 48);
+    return std::max(1, std::min(4, per));
+}
+
+// The ingest pass (16 or 8 columns wide) for `remaining` columns, or 0: the widest whose stage fits kWideStageBytes (16
+// also in two K halves) and that saves a pass - 16 from 9 columns on, 8 once the columns are more than one narrow pass
+// takes.  A part-full pass stages its last column in the missing ones' place and stores nothing for them: 4096 x 12352
+// with 5 columns 23.1 -> 15.5 us (4 + 1 before), 9 columns 24.0 -> 20.0 (8 + 1), 15 columns 40.7 -> 20.1 (8 + 4 + 3);
+// 12288 x 4096 with 4 columns 22.0 -> 17.4 (3 + 1).  One narrow pass stays the faster one (3 / 4 columns 13.4 / 14.6).
 int wide_cols(int n_in, int n_out, int remaining) {
-    if (remaining >= 16 && (wide_stage_bytes(n_in, 16) <= kWideStageBytes || wide_halves(n_in, n_out))) return 16;
-    if (remaining >= 8 && wide_stage_bytes(n_in, 8) <= kWideStageBytes) return 8;
+    if (remaining > 8 && (wide_stage_bytes(n_in, 16) <= kWideStageBytes || wide_halves(n_in, n_out))) return 16;
+    if (remaining > cols_per_pass(n_in) && wide_stage_bytes(n_in, 8) <= kWideStageBytes) return 8;
     return 0;
 }
 
-// 8 / 16 columns in one weight pass on the MFMA ingest kernel: one 8-wave workgroup per CU (the stage takes up to
+// Up to 8 / 16 columns in one weight pass on the MFMA ingest kernel: one 8-wave workgroup per CU (the stage takes up to
 // 160 KB of LDS), the quads split evenly over the waves
 // workgroups of a grid whose quad units (one per wave, or per pair of waves at CS = 2) spread evenly over the CUs
 int wide_grid(int nq, int units_per_wg) {
@@ -1331,7 +1341,7 @@ int wide_grid(int nq, int units_per_wg) {
 
 template <int NCOLS, bool RES>
 int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const float* res, float* partials, int n_in,
-                       int n_out, hipStream_t s) {
+                       int n_out, int ncols, hipStream_t s) {
     constexpr int D = 3;
     constexpr int NCG = NCOLS / 4;
     auto kern = q6k_packed_mfma<NCG, RES, D>;
@@ -1361,9 +1371,9 @@ int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const floa
                 const dim3 grid((nq + kWideWaves / 2 - 1) / (kWideWaves / 2)), block(64 * kWideWaves);
                 if (lds / 2 < le_bytes(2)) return fail(RMI_ERR_SHAPE, "native_q6_k_mmvq_packed: half stage too small");
                 if (n_in / kChunkElems == 4)
-                    hipLaunchKernelGGL(kh4, grid, block, lds / 2, s, wp, x, y, res, partials, n_in, n_out);
+                    hipLaunchKernelGGL(kh4, grid, block, lds / 2, s, wp, x, y, res, partials, n_in, n_out, ncols);
                 else if (n_in / kChunkElems == 6)
-                    hipLaunchKernelGGL(kh6, grid, block, lds / 2, s, wp, x, y, res, partials, n_in, n_out);
+                    hipLaunchKernelGGL(kh6, grid, block, lds / 2, s, wp, x, y, res, partials, n_in, n_out, ncols);
                 else
                     return fail(RMI_ERR_SHAPE, "native_q6_k_mmvq_packed: wide stage exceeds the LDS");
                 return RMI_OK;
@@ -1379,26 +1389,20 @@ int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const floa
     if (split_on && 4 * g1 < 3 * cu_count() && g2 > g1) {
         const size_t l2 = lds + le_bytes(NCG / 2);
         if (le_on && NCG >= 2 && l2 <= kWideStageBytes)
-            hipLaunchKernelGGL(kern2l, dim3(g2), block, l2, s, wp, x, y, res, partials, n_in, n_out);
+            hipLaunchKernelGGL(kern2l, dim3(g2), block, l2, s, wp, x, y, res, partials, n_in, n_out, ncols);
         else
-            hipLaunchKernelGGL(kern2, dim3(g2), block, lds, s, wp, x, y, res, partials, n_in, n_out);
+            hipLaunchKernelGGL(kern2, dim3(g2), block, lds, s, wp, x, y, res, partials, n_in, n_out, ncols);
     } else {
         const size_t l1 = lds + le_bytes(NCG);
         if (le_on && l1 <= kWideStageBytes)
-            hipLaunchKernelGGL(kernl, dim3(g1), block, l1, s, wp, x, y, res, partials, n_in, n_out);
+            hipLaunchKernelGGL(kernl, dim3(g1), block, l1, s, wp, x, y, res, partials, n_in, n_out, ncols);
         else
-            hipLaunchKernelGGL(kern, dim3(g1), block, lds, s, wp, x, y, res, partials, n_in, n_out);
+            hipLaunchKernelGGL(kern, dim3(g1), block, lds, s, wp, x, y, res, partials, n_in, n_out, ncols);
     }
     return RMI_OK;
 }
 
-// columns per narrow pass: at most 4, and the pass's staged activations within kMaxStageBytes
-int cols_per_pass(int n_in) {
-    const int per = kMaxStageBytes / ((n_in / 32) * 48);
-    return std::max(1, std::min(4, per));
-}
-
-// Columns are cut into passes (16 or 8 wide, then up to 4); each pass reads the weights once.  The pass width never
+// Columns are cut into passes (up to 16 or 8 on the ingest kernel, up to 4 on the others); each pass reads the weights once.  The pass width never
 // changes a column's result: lane ownership and reduction order depend on the shape only.
 template <bool RES>
 int run_packed(const void* wpv, const void* xv, float* y, const float* res, float* partials, int n_in, int n_out,
@@ -1410,22 +1414,22 @@ int run_packed(const void* wpv, const void* xv, float* y, const float* res, floa
     const size_t pcol = static_cast<size_t>((n_out + 3) / 4);
     for (int j = 0; j < ncols;) {
         const int wide = wide_cols(n_in, n_out, ncols - j);
-        const int nj = wide ? wide : std::min(per, ncols - j);
+        const int nj = std::min(wide ? wide : per, ncols - j);
         const uint8_t* xj = x + j * xcol;
         float* yj = y + static_cast<size_t>(j) * n_out;
         const float* rj = RES ? res + static_cast<size_t>(j) * n_out : nullptr;
         float* pj = RES ? partials + j * pcol : nullptr;
-        switch (nj) {
-            case 1: launch_packed<1, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
-            case 2: launch_packed<2, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
-            case 3: launch_packed<3, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
-            case 4: launch_packed<4, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
-            case 8:
-                if (const int rc = launch_packed_wide<8, RES>(wp, xj, yj, rj, pj, n_in, n_out, s)) return rc;
-                break;
-            default:
-                if (const int rc = launch_packed_wide<16, RES>(wp, xj, yj, rj, pj, n_in, n_out, s)) return rc;
-                break;
+        if (wide) {
+            const int rc = wide == 8 ? launch_packed_wide<8, RES>(wp, xj, yj, rj, pj, n_in, n_out, nj, s)
+                                     : launch_packed_wide<16, RES>(wp, xj, yj, rj, pj, n_in, n_out, nj, s);
+            if (rc) return rc;
+        } else {
+            switch (nj) {
+                case 1: launch_packed<1, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
+                case 2: launch_packed<2, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
+                case 3: launch_packed<3, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
+                default: launch_packed<4, RES>(wp, xj, yj, rj, pj, n_in, n_out, s); break;
+            }
         }
         if (const int rc = launch_status("native_q6_k_mmvq_packed")) return rc;
         j += nj;
