@@ -75,11 +75,11 @@ int rmi_engine_create(const rmi_model_config* cfg, uint64_t seed, int max_ctx, v
 int rmi_engine_destroy(rmi_engine* e);
 int rmi_engine_info(const rmi_engine* e, rmi_engine_info_t* info);
 /* prompt of n host tokens from position 0; *first_out = the greedy token after it (the current token).  Ingests in
- * chunks of 16 tokens (rmi_engine_prefill_batch with batch 16). */
+ * chunks (rmi_engine_prefill_batch with batch 16). */
 int rmi_engine_prefill(rmi_engine* e, const int* tokens, int n, int* first_out);
 /* batch 1: token by token (forward_token per prompt token, qw:1773-1824, plus the draft KV row); batch 2..16: chunks
- * of `batch` tokens, one weight pass per chunk (serve_ingest_kernels, qw:2192-2502, the batch loop qw:2658-2722; the
- * reference takes 2..8 or 16).  Every batch leaves the same state, bit for bit: GDN state and history, trunk and
+ * of `batch` tokens, one weight pass per chunk, at 16 of up to 1024 tokens while 64 or more are left and every matrix is
+ * packed (serve_ingest_kernels, qw:2192-2502, the batch loop qw:2658-2722; the reference takes 2..8 or 16).  Every batch leaves the same state, bit for bit: GDN state and history, trunk and
  * draft KV, hidden, position and first token. */
 int rmi_engine_prefill_batch(rmi_engine* e, const int* tokens, int n, int batch, int* first_out);
 /* seeded synthetic state for positions [0, n_ctx - 1), then one forward of last_token at n_ctx - 1 */

@@ -30,7 +30,7 @@ constexpr int HD = 256;
 constexpr int SUB = 64;            // positions per chunk unit (4 waves x 16); a chunk is SUB * nsub positions
 constexpr int REC = HD + 4;        // workspace record: m, l, pad, pad, o[256]
 constexpr int SLOTS = 8;           // query vectors per kv head one partial workgroup handles (tokens x group heads)
-constexpr int kMaxSlots = 64;      // query vectors per kv head one launch handles: SLOTS per slot group, grid.z groups
+constexpr int kMaxSlots = 64;      // query vectors per kv head one launch handles: SLOTS per slot group
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));

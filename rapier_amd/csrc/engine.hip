@@ -1408,7 +1408,7 @@ extern "C" int rmi_engine_reset(rmi_engine* h) {
 // qw:2956-2958) and every later slot with (token, previous final-normed hidden).  batch 1: one token at a time (the
 // trunk with its head, then the draft row, per token; forward_token, qw:1773-1824).  batch 2..16: chunks of `batch`
 // tokens, each one pass over the weights (the ingest of qw:2658-2722), the head on the last token only; a full chunk is
-// one hipGraph launch.  Both leave the same state.  *first_out = the greedy token after the last one fed (the current
+// one hipGraph launch, and at 16 wide chunks go first.  Both leave the same state.  *first_out = the greedy token after the last one fed (the current
 // token).  After a generation the context continues at its position, as the reference's serve loop does.
 extern "C" int rmi_engine_ingest(rmi_engine* h, const int* tokens, int n, int batch, int* first_out) {
     if (!h || !tokens) return fail(RMI_ERR_POINTER, "rmi_engine_ingest: null argument");

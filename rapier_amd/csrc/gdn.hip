@@ -1,8 +1,8 @@
 // gdn.hip - Gated DeltaNet decode chain for gfx950 (reference src/fused_gdn.cu:40-133, engine glue
 // src/qwythos.cpp:1101-1127 and the verify pass 1438-1478).
 //
-// Kernels, for 1 token (the plain decode step), the 2 verify tokens or an ingest chunk of up to 16 tokens (the engine
-// path runs the conv inside the step kernel's prologue, one launch per layer; the reference surface keeps them apart):
+// Kernels, for 1 token (the plain decode step) or the 2 verify tokens (longer chunks: gdn_chunk_* and gdn_wide_* below;
+// the engine path runs the conv inside the step kernel's prologue, one launch per layer; the reference surface keeps them apart):
 //   conv:  one lane per channel (8192 = q 2048 | k 2048 | v 4096): causal width-4 conv over [hist(3) | x], SiLU, and
 //          the L2 norm of each 128-channel q/k head.  History is updated in place; with 2 tokens the history after
 //          token 0 also goes to the rollback buffer.
@@ -122,9 +122,9 @@ struct StepArgs {
 // q|k|v rows are only read.
 //
 // NT is the largest token count of the instantiation and a.ntok (<= NT) the count of this launch.  NT = 2 is the
-// verify pair: the state and history after token 0 also go to the rollback buffers.  Otherwise (1 token, or an ingest
-// chunk of up to 16) the state and history are updated in place after the last token.  Every token's arithmetic is
-// that of the single-token step in the same order, so a chunk leaves the bits the per-token steps leave.
+// verify pair: the state and history after token 0 also go to the rollback buffers.  Otherwise the state and history are
+// updated in place after the last token.  Every token's arithmetic is that of the single-token step in the same order,
+// so a pair leaves the bits the per-token steps leave.
 // v[l] + v[l ^ 16], then that plus its value in lane l ^ 32: the sum over a column's four row groups, in every lane of
 // the column.  gfx950's lane swaps (v_permlane16_swap / v_permlane32_swap: each returns a half's even / odd rows, or
 // the two 32-lane halves, side by side) keep it on the VALU; the sums are those of the xor-16 / xor-32 butterfly
@@ -154,7 +154,7 @@ __device__ __forceinline__ void gate_values(float b_raw, float a_raw, float dt, 
 template <int NT, bool RAW, bool CONV>
 __global__ __launch_bounds__(S * RG) void gdn_step_kernel(StepArgs a) {
     constexpr bool SNAP = NT == 2;
-    // the engine path (decode, verify, ingest chunks): the launch's loads go out in one batch led by the selector
+    // the engine path (decode, verify): the launch's loads go out in one batch led by the selector
     // (both history buffers read, one kept), so the state loads wait for one memory round trip, not three; the gates
     // are derived by the conv's idle lanes and published by the conv's own barrier
     constexpr bool FAST = CONV && RAW;
@@ -786,7 +786,7 @@ __device__ __forceinline__ float4 scan_outputs(const float* part, int ln, float&
 // writes the conv history, which the first launch's four parts all read.  In a part the four waves share the conv (waves
 // 0, 1 the head's q channels, 2, 3 its k channels, all four the part's v), and waves 0, 1 then run the recurrence on 16
 // columns each.  One workgroup per value head (gdn_step_kernel) had its eight waves queue for the same LDS rows:
-// 16 tokens of the 9B layer 20.9 us; this pair MEASURED.
+// 16 tokens of the 9B layer 20.9 us; this pair 15.2 us.
 constexpr int kChunkTok = kMaxCols;
 
 __global__ __launch_bounds__(2 * S) void gdn_chunk_scan(StepArgs a) {
