@@ -931,7 +931,7 @@ __global__ __launch_bounds__(S) void gdn_chunk_finish(StepArgs a) {
 // wave here), so the bits are those of the per-token steps.
 // The scan is bound by its own vector instructions, 128 per token and lane (mul, two fmas of the update and output, one
 // fma of the next token's S^T k, which rides along so that the two chains hide each other's latency); 256 waves of the
-// 9B shape, one per CU.  1000 tokens of a 9B layer: 608 us (prep 17, scan 574, finish 17) where 62.5 launches of the
+// 9B shape, one per CU.  1000 tokens of a 9B layer: 416 us (prep 17, scan 382, finish 17) where 62.5 launches of the
 // 16-token kernel take 1410 us.
 constexpr int kScanTok = 16;   // tokens staged per step, double-buffered
 
