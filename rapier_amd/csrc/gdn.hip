@@ -1,8 +1,9 @@
 // gdn.hip - Gated DeltaNet decode chain for gfx950 (reference src/fused_gdn.cu:40-133, engine glue
 // src/qwythos.cpp:1101-1127 and the verify pass 1438-1478).
 //
-// Kernels, for 1 token (the plain decode step) or the 2 verify tokens (longer chunks: gdn_chunk_* and gdn_wide_* below;
-// the engine path runs the conv inside the step kernel's prologue, one launch per layer; the reference surface keeps them apart):
+// Kernels, for 1 token (the plain decode step), the 2 verify tokens or a chunk of up to 16 tokens (most chunks:
+// gdn_chunk_* and gdn_wide_* below).  The layer call runs the conv inside the step kernel's prologue, one launch per
+// layer; the reference surface keeps them apart:
 //   conv:  one lane per channel (8192 = q 2048 | k 2048 | v 4096): causal width-4 conv over [hist(3) | x], SiLU, and
 //          the L2 norm of each 128-channel q/k head.  History is updated in place; with 2 tokens the history after
 //          token 0 also goes to the rollback buffer.
@@ -124,7 +125,7 @@ struct StepArgs {
 // NT is the largest token count of the instantiation and a.ntok (<= NT) the count of this launch.  NT = 2 is the
 // verify pair: the state and history after token 0 also go to the rollback buffers.  Otherwise the state and history are
 // updated in place after the last token.  Every token's arithmetic is that of the single-token step in the same order,
-// so a pair leaves the bits the per-token steps leave.
+// so a pair or a chunk leaves the bits the per-token steps leave.
 // v[l] + v[l ^ 16], then that plus its value in lane l ^ 32: the sum over a column's four row groups, in every lane of
 // the column.  gfx950's lane swaps (v_permlane16_swap / v_permlane32_swap: each returns a half's even / odd rows, or
 // the two 32-lane halves, side by side) keep it on the VALU; the sums are those of the xor-16 / xor-32 butterfly
@@ -154,7 +155,7 @@ __device__ __forceinline__ void gate_values(float b_raw, float a_raw, float dt, 
 template <int NT, bool RAW, bool CONV>
 __global__ __launch_bounds__(S * RG) void gdn_step_kernel(StepArgs a) {
     constexpr bool SNAP = NT == 2;
-    // the engine path (decode, verify): the launch's loads go out in one batch led by the selector
+    // the layer call: the launch's loads go out in one batch led by the selector
     // (both history buffers read, one kept), so the state loads wait for one memory round trip, not three; the gates
     // are derived by the conv's idle lanes and published by the conv's own barrier
     constexpr bool FAST = CONV && RAW;
@@ -1181,6 +1182,11 @@ int gdn_layer(float* state_a, float* state_b, float* hist_a, float* hist_b, cons
     a.hist_a = hist_a; a.hist_b = hist_b; a.conv_w = conv_w;
     a.ntok = ntok;
     a.xch = static_cast<unsigned long long*>(xch);
+    // the chunk kernels carry raw outputs through y and read z and the last q|k|v rows behind it; a y laid over those
+    // rows, or whose own rows overlap, takes the one-workgroup kernel, which has read its inputs before it writes
+    const float* y_end = y + static_cast<ptrdiff_t>(ntok - 1) * y_stride + h_v * S;
+    const float* in_end = qkvz + static_cast<ptrdiff_t>(ntok - 1) * qkvz_stride + channels + h_v * S;
+    const bool apart = y_stride >= h_v * S && (y_end <= qkvz || in_end <= y);
     if (ntok <= 2 && xch) {
         // decode / verify: four workgroups per value head (bitwise the one-workgroup kernel)
         if (ntok == 2) hipLaunchKernelGGL((gdn_split_kernel<2>), dim3(h_v * kParts), dim3(kPartLanes), 0, s, a);
@@ -1189,6 +1195,8 @@ int gdn_layer(float* state_a, float* state_b, float* hist_a, float* hist_b, cons
         hipLaunchKernelGGL((gdn_step_kernel<2, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
     } else if (ntok == 1) {
         hipLaunchKernelGGL((gdn_step_kernel<1, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
+    } else if (!apart) {
+        hipLaunchKernelGGL((gdn_step_kernel<kMaxCols, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
     } else {
         hipLaunchKernelGGL(gdn_chunk_scan, dim3(h_v * kParts), dim3(2 * S), 0, s, a);
         hipLaunchKernelGGL(gdn_chunk_finish, dim3(h_v, ntok), dim3(S), 0, s, a);

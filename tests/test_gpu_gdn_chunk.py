@@ -47,3 +47,43 @@ def test_chunk_is_its_single_steps(h_k, h_v, ntok, sel, q8):
 
     for u, v in zip(run(ntok), run(1)):
         assert T.equal(u, v)
+
+
+@pytest.mark.parametrize("over,h_k,h_v,ntok", [("z", 16, 32, 16), ("z", 3, 6, 7), ("v", 16, 32, 9), ("v", 2, 4, 16),
+                                               ("one row", 4, 8, 8)])
+def test_chunk_output_over_its_inputs(over, h_k, h_v, ntok):
+    """y laid over the z or v rows, or one y row for every token (only its Q8_1 wanted): the same results"""
+    import rapier_amd as rmi
+    from tests.gpu_util import torch
+    T = torch()
+    g = T.Generator(device="cuda")
+    g.manual_seed(h_v)
+    rnd = lambda *s, std=1.0: T.randn(*s, generator=g, device="cuda") * std  # noqa: E731
+    ch = 2 * h_k * S + h_v * S
+    row = ch + h_v * S
+    x0, ab = rnd(ntok, row), rnd(ntok, 2 * h_v)
+    conv_w, dt = rnd(ch, 4, std=0.5), rnd(h_v, std=0.1)
+    ssm_a, gamma = -T.exp(rnd(h_v, std=0.5)), 1 + rnd(S, std=0.1)
+    state0, hist0 = rnd(S, h_v, S, std=0.05), rnd(h_v, 3, S, 3, std=0.5)
+    st = T.cuda.Stream()
+    sel = T.zeros(1, dtype=T.int32, device="cuda")
+
+    def run(y_of):
+        x, live, hist = x0.clone(), state0.clone(), hist0.clone()
+        y, stride = y_of(x)
+        o = T.zeros(ntok, h_v * S // 32 * 36, dtype=T.uint8, device="cuda")
+        T.cuda.synchronize()
+        rmi.gdn_layer_tokens(live, T.zeros_like(live), hist, T.zeros_like(hist), sel, x, row, ab, 2 * h_v, conv_w, dt, ssm_a,
+                             gamma, EPS, y, stride, o, o.shape[1], h_k, h_v, ntok, stream=st)
+        T.cuda.synchronize()
+        return y, o, live, hist
+
+    ref = run(lambda x: (T.zeros(ntok, h_v * S, device="cuda"), h_v * S))
+    if over == "one row":
+        got = run(lambda x: (T.zeros(h_v * S, device="cuda"), 0))
+    else:
+        at = ch if over == "z" else 2 * h_k * S
+        got = run(lambda x: (x[:, at:at + h_v * S], row))
+        assert T.equal(got[0], ref[0])
+    for u, v in zip(got[1:], ref[1:]):
+        assert T.equal(u, v)
