@@ -1,7 +1,7 @@
 // gdn.hip - Gated DeltaNet decode chain for gfx950 (reference src/fused_gdn.cu:40-133, engine glue
 // src/qwythos.cpp:1101-1127 and the verify pass 1438-1478).
 //
-// Kernels, for 1 token (the plain decode step), the 2 verify tokens or a chunk of up to 16 tokens (most chunks:
+// Kernels, for 1 token (the plain decode step), the 2 verify tokens or a chunk of 3..5 tokens (longer ones:
 // gdn_chunk_* and gdn_wide_* below).  The layer call runs the conv inside the step kernel's prologue, one launch per
 // layer; the reference surface keeps them apart:
 //   conv:  one lane per channel (8192 = q 2048 | k 2048 | v 4096): causal width-4 conv over [hist(3) | x], SiLU, and
@@ -781,14 +781,17 @@ __device__ __forceinline__ float4 scan_outputs(const float* part, int ln, float&
     return make_float4(oc[0], oc[1], oc[2], oc[3]);
 }
 
-// ---- ingest chunks of 3..16 tokens: four workgroups per value head, then the output norm -----------------------------
+// ---- ingest chunks of 6..16 tokens: four workgroups per value head, then the output norm -----------------------------
 // A chunk's first launch holds each value head's 128 state columns in four parts of 32, as the split kernel does, but
 // leaves the raw outputs in y; the second takes the norm over the head's columns, the gate and the Q8_1 blocks, and
 // writes the conv history, which the first launch's four parts all read.  In a part the four waves share the conv (waves
 // 0, 1 the head's q channels, 2, 3 its k channels, all four the part's v), and waves 0, 1 then run the recurrence on 16
 // columns each.  One workgroup per value head (gdn_step_kernel) had its eight waves queue for the same LDS rows:
-// 16 tokens of the 9B layer 20.9 us; this pair 15.2 us.
+// 16 tokens of the 9B layer 20.9 us; this pair 14.6 us.  The second launch and the raw outputs' way through memory cost
+// ~2.5 us, which chunks of 3..5 tokens do not win back (16 / 32 heads, one workgroup per head against this pair: 3 tokens
+// 8.6 / 10.2 us, 4 9.5 / 10.6, 5 10.5 / 11.0, 6 11.5 / 11.2, 8 13.4 / 12.0; 1 / 2 to 16 / 64 heads alike).
 constexpr int kChunkTok = kMaxCols;
+constexpr int kChunkMin = 6;
 
 __global__ __launch_bounds__(2 * S) void gdn_chunk_scan(StepArgs a) {
     __shared__ __attribute__((aligned(16))) float cqk[2][kChunkTok][S];   // q and k, convolved and normalized
@@ -1195,7 +1198,7 @@ int gdn_layer(float* state_a, float* state_b, float* hist_a, float* hist_b, cons
         hipLaunchKernelGGL((gdn_step_kernel<2, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
     } else if (ntok == 1) {
         hipLaunchKernelGGL((gdn_step_kernel<1, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
-    } else if (!apart) {
+    } else if (ntok < kChunkMin || !apart) {
         hipLaunchKernelGGL((gdn_step_kernel<kMaxCols, true, true>), dim3(h_v), dim3(S * RG), 0, s, a);
     } else {
         hipLaunchKernelGGL(gdn_chunk_scan, dim3(h_v * kParts), dim3(2 * S), 0, s, a);

@@ -1,5 +1,5 @@
-"""Chunks of 3..16 tokens on four workgroups per value head: the bits of the single-token steps for head counts that are
-no multiple of eight, the second buffer live, rows wider than their data, and no Q8_1 output."""
+"""Chunks of 3..5 tokens on one workgroup per value head and of 6..16 on four: the bits of the single-token steps for head
+counts that are no multiple of eight, the second buffer live, rows wider than their data, and no Q8_1 output."""
 import ctypes
 
 import numpy as np
@@ -10,7 +10,7 @@ S, EPS = 128, 1e-6
 
 
 @pytest.mark.parametrize("h_k,h_v,ntok,sel,q8", [(1, 2, 3, 0, True), (3, 6, 4, 1, True), (6, 6, 15, 1, False), (2, 8, 16, 0, True),
-                                                 (16, 32, 5, 1, True)])
+                                                 (16, 32, 5, 1, True), (2, 4, 6, 1, True), (5, 10, 7, 0, True)])
 def test_chunk_is_its_single_steps(h_k, h_v, ntok, sel, q8):
     import rapier_amd as rmi
     from tests.gpu_util import torch
