@@ -431,20 +431,51 @@ int pick(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* 
     return go(launch<TYPE, NLU, 6, false>, launch<TYPE, NLU, 6, true>);
 }
 
-// The fewest columns from which this kernel beats passes of at most four over the weights (measured, this kernel
-// against the passes, us):
-//   nine columns on: everywhere measured (Q4_K 4096 x 512 8.3 / 8.6, 24576 x 4096 24 / 49; at 16 columns 8.4 / 12.3, 25 / 78)
-//   five to eight (two passes): K-quants from ~9M weights (2048 x 4096 at 5: 8.5 / 7.2, 4096 x 2304 8.0 / 8.2, 4096 x
-//   4096 9.1 / 9.1, at 8: 9.1 / 11.2), Q8_0 from ~8M (4096 x 512 8.1 / 7.0, 2048 x 4096 8.5 / 9.8), Q6_K except rows above
-//   8192 (4096 x 12288 at 8: 27.6 / 26.9)
-//   three and four (one pass): Q6_K rows the streaming kernels do not take (20000 x 1024 16 / 33, 4096 x 2304 8.4 / 10.4)
-//   and large Q8_0 matrices (24576 x 4096 26 / 39, 10240 x 4096 16.4 / 18.4, 4096 x 4096 9.5 / 9.0)
-int cols_min(int type, int lanes, int n_in, int n_out) {
-    const int64_t weights = static_cast<int64_t>(n_in) * n_out;
-    if (type == 12 || type == 13) return weights >= 9000000 ? 5 : 9;
-    if (type == 8) return weights >= 32000000 ? 3 : weights >= 8000000 ? 5 : 9;
-    if (lanes == 64) return weights >= 8000000 ? 3 : 5;
-    return n_in > 8192 ? 9 : 5;
+// The fewest rows from which this kernel beats passes of at most four columns over the weights.  A launch's time steps
+// with its tiles per workgroup (one per 4096 rows) and hardly depends on its columns; a pass's grows with the rows from
+// the first one on, so few columns, and few rows of a long row's prologue, stay with the passes.  From grids of 64 to
+// 24576 rows (this kernel / the passes, us):
+//   Q4_K 6144 wide, 5 columns: 2048 rows 12.6 / 8.9, 7168 17.1 / 17.9; 8 columns: 2048 12.8 / 11.0, 3072 12.9 / 13.5
+//   Q4_K 12288 wide, 5 columns: 1024 rows 18.6 / 9.7, 4608 25.5 / 25.1; 12 columns: 1024 18.8 / 17.2, 1280 19.0 / 23.3
+//   Q6_K off the streaming shapes, 3 columns: 11008 wide 1024 rows 23.2 / 7.9, 5632 36.3 / 38.2; 1024 wide 2048 rows
+//     6.7 / 5.4, 2560 6.8 / 7.0; 8 columns: 11008 wide 1024 rows 23.4 / 19.5, 1280 23.7 / 29.0
+//   Q6_K on them: 3 and 4 columns slower everywhere, 8 faster everywhere to 8192 wide
+//   Q8_0 12288 wide, 5 columns: 1024 rows 16.5 / 12.8, 1280 16.6 / 19.6; 3 columns: 5120 26.8 / 26.4, 5632 27.0 / 30.3
+constexpr int kNever = 1 << 30;
+struct Line {
+    int max_in;    // rows of at most this length
+    int rows[8];   // at 3, 4, .., 9 and 10..12 columns; from 13 on any
+};
+constexpr Line kLinesK[] = {{1024, {kNever, kNever, 2560, 2560, 1280, 1280, 0, 0}},
+                            {2048, {kNever, kNever, 5632, 5632, 2560, 2560, 0, 0}},
+                            {4096, {kNever, kNever, 10240, 6144, 5120, 4608, 768, 0}},
+                            {10240, {kNever, kNever, 7168, 5632, 3584, 2560, 1280, 1280}},
+                            {12288, {kNever, kNever, 4608, 2560, 2560, 2560, 1280, 1280}}};
+constexpr Line kLinesQ8[] = {{2048, {kNever, kNever, 5632, 5120, 2560, 2560, 0, 0}},
+                             {4096, {10240, 5632, 1280, 1280, 1280, 1280, 0, 0}},
+                             {8192, {10240, 5632, 2048, 1280, 1280, 1280, 0, 0}},
+                             {12288, {5632, 3584, 1280, 1280, 1280, 1280, 768, 0}}};
+constexpr Line kLinesQ6[] = {{1024, {2560, 1280, 0, 0, 0, 0, 0, 0}},   // 64 lanes
+                             {2048, {5632, 2560, 0, 0, 0, 0, 0, 0}},
+                             {4096, {5632, 2560, 1280, 1280, 0, 0, 0, 0}},
+                             {8192, {10240, 4608, 2560, 1536, 1280, 1280, 0, 0}},
+                             {12288, {5632, 3584, 1536, 1280, 1280, 1280, 256, 0}}};
+constexpr Line kLinesQ6Stream[] = {{2048, {kNever, kNever, kNever, kNever, kNever, 0, 0, 0}},   // 16 lanes
+                                   {6144, {kNever, kNever, 512, 0, 0, 0, 0, 0}},
+                                   {8192, {kNever, kNever, 2048, 0, 0, 0, 0, 0}},
+                                   {12288, {kNever, kNever, kNever, kNever, kNever, kNever, 0, 0}}};
+
+template <int N>
+int rows_min(const Line (&lines)[N], int n_in, int ncols) {
+    for (const Line& l : lines)
+        if (n_in <= l.max_in) return ncols >= 13 ? 0 : l.rows[std::min(ncols, 10) - 3];
+    return kNever;
+}
+
+int rows_min(int type, int lanes, int n_in, int ncols) {
+    if (type == 12 || type == 13) return rows_min(kLinesK, n_in, ncols);
+    if (type == 8) return rows_min(kLinesQ8, n_in, ncols);
+    return lanes == 16 ? rows_min(kLinesQ6Stream, n_in, ncols) : rows_min(kLinesQ6, n_in, ncols);
 }
 
 }  // namespace
@@ -454,7 +485,7 @@ int cols_gemv(int type, int lanes, const uint8_t* w, const uint8_t* x, float* y,
     if (ncols > 16 || n_in > 12288 || n_in % 256 ||
         static_cast<uint64_t>(n_out) * (n_in / 32) * kQ8_0Bytes >= (uint64_t(1) << 32))
         return -1;
-    if (ncols < cols_min(type, lanes, n_in, n_out)) return -1;
+    if (ncols < 3 || n_out < rows_min(type, lanes, n_in, ncols)) return -1;
     if (type == 12) return pick<12, 16>(w, x, y, res, partials, n_in, n_out, ncols, s);
     if (type == 13) return pick<13, 16>(w, x, y, res, partials, n_in, n_out, ncols, s);
     if (type == 8) return (reinterpret_cast<uintptr_t>(w) & 1) ? -1 : pick<8, 8>(w, x, y, res, partials, n_in, n_out, ncols, s);

@@ -1,5 +1,6 @@
 """The one-pass GEMV over several columns (mmvq_cols.hip) gives the single-column kernel's bits: rows that end inside a
-slab, tiles with rows and columns missing, one to six slabs, several tiles per workgroup, every lane split of Q6_K."""
+slab, tiles with rows and columns missing, one to six slabs, several tiles per workgroup, both lane splits of Q6_K at each
+of them, and the fewest columns and rows each type takes it from (with the calls just below, which keep the passes)."""
 import ctypes
 
 import numpy as np
@@ -21,11 +22,15 @@ def blocks(oracle, name, n_out, n_in, seed):
     return b.reshape(-1)
 
 
-@pytest.mark.parametrize("name", list(TYPES))
+# off 4: a matrix 4 bytes off 16 (Q6_K: off its streaming kernels)
+@pytest.mark.parametrize("name,off", [(n, 0) for n in TYPES] + [("q6_k", 4), ("q8_0", 4)])
 @pytest.mark.parametrize("n_in,n_out,ncols,res", [
     (256, 17, 9, True), (1280, 33, 16, False), (2048, 40, 12, True), (4096, 2051, 5, False), (4096, 4300, 16, True),
-    (6144, 70, 13, True), (8192, 1100, 8, False), (11008, 50, 11, False), (12288, 16, 16, True), (12288, 100, 9, False)])
-def test_columns_are_the_single_column_bits(name, n_in, n_out, ncols, res):
+    (6144, 70, 13, True), (8192, 1100, 8, False), (11008, 50, 11, False), (12288, 16, 16, True), (12288, 100, 9, False),
+    (768, 2560, 5, True), (768, 2559, 5, False), (1024, 2561, 3, True), (5120, 1700, 3, False), (5120, 70, 13, True),
+    (5120, 5000, 4, False), (4096, 8200, 3, True), (4096, 10241, 5, False), (3072, 10240, 3, False), (4096, 5700, 4, True),
+    (12288, 4608, 5, False), (12288, 5633, 3, True)])
+def test_columns_are_the_single_column_bits(name, n_in, n_out, ncols, res, off):
     import oracle
     import rapier_amd as rmi
     from tests.gpu_util import torch
@@ -34,7 +39,7 @@ def test_columns_are_the_single_column_bits(name, n_in, n_out, ncols, res):
     st = T.cuda.Stream()
     h = ctypes.c_void_p(st.cuda_stream)
     dev = lambda a: T.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
-    w = dev(blocks(oracle, name, n_out, n_in, n_out))
+    w = dev(np.concatenate([np.zeros(off, np.uint8), blocks(oracle, name, n_out, n_in, n_out)]))[off:]
     q = n_in // 32 * 36
     xq = dev(oracle.quantize_q8_1(oracle.normal(n_in * ncols, seed=n_in), n_in, ncols))
     np_ = (n_out + 3) // 4
