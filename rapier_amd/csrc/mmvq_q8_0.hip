@@ -214,21 +214,26 @@ void launch_staged(const uint8_t* w, const uint8_t* x, float* y, const float* re
 // more than 10M elements.  Below that the two-byte loads are faster, their chain being shorter (no LDS behind the loads):
 // 2048 x 4096 3.8 us against 4.3, 12288 x 512 4.6 / 5.1; above it 4096 x 3072 6.6 / 5.1, 12288 x 1024 6.6 / 5.8,
 // 4096 x 24576 33.2 / 21.4 (one column; two columns alike).  Short rows leave its lanes idle: 512 x 16384 5.6 / 7.3.
-bool staged(const uint8_t* w, const uint8_t* x, int n_in, int n_out, int ncols) {
-    return n_in >= 2048 && n_in % 256 == 0 && static_cast<int64_t>(n_in) * n_out > 10000000 && aligned16(w) && aligned16(x) &&
+// At 2048 wide the line is 11M: 4900 rows (10.0M) 4.9 / 5.1, 5632 (11.5M) 5.5 / 5.2.  As the last pass of a call of more
+// columns (`behind`) it finds the weights in the caches, which the two-byte loads use better where workgroups or steps are
+// few: the whole call of five columns 2048 x 4900 10.4 / 11.7, 10240 x 1024 11.3 / 11.7, 20480 x 1024 (six) 19.6 / 20.0,
+// but 8192 x 1300 14.3 / 13.7, 12288 x 1279 19.8 / 18.6, 20480 x 4096 56.2 / 53.8.
+bool staged(const uint8_t* w, const uint8_t* x, int n_in, int n_out, int ncols, bool behind) {
+    return n_in >= 2048 && n_in % 256 == 0 && static_cast<int64_t>(n_in) * n_out > (n_in > 2048 ? 10000000 : 11000000) &&
+           (!behind || (n_in >= 4096 && n_out >= 1280)) && aligned16(w) && aligned16(x) &&
            static_cast<int64_t>(ncols) * (n_in / 32) * kQ8_1Bytes <= kStagedMax;
 }
 
 template <bool RES>
 int launch(const void* wv, const void* xv, float* y, const float* res, float* partials, int n_in, int n_out,
-           int ncols, hipStream_t s) {
+           int ncols, hipStream_t s, bool behind = false) {
     const auto* w = static_cast<const uint8_t*>(wv);
     const auto* x = static_cast<const uint8_t*>(xv);
     const dim3 grid((n_out + 3) / 4), block(256);
     if (ncols > 2)
         if (const int rc = cols_gemv(8, 64, w, x, y, res, partials, n_in, n_out, ncols, s); rc >= 0)
             return rc;
-    if (ncols <= 2 && staged(w, x, n_in, n_out, ncols)) {
+    if (ncols <= 2 && staged(w, x, n_in, n_out, ncols, behind)) {
         if (ncols == 1) launch_staged<1, RES>(w, x, y, res, partials, n_in, n_out, s);
         else launch_staged<2, RES>(w, x, y, res, partials, n_in, n_out, s);
         return launch_status("native_q8_0_mmvq");
@@ -240,7 +245,7 @@ int launch(const void* wv, const void* xv, float* y, const float* res, float* pa
             const int nj = ncols - j < 4 ? ncols - j : 4;
             const int rc = launch<RES>(w, x + j * xcol, y + static_cast<size_t>(j) * n_out,
                                        RES ? res + static_cast<size_t>(j) * n_out : nullptr,
-                                       RES ? partials + j * pcol : nullptr, n_in, n_out, nj, s);
+                                       RES ? partials + j * pcol : nullptr, n_in, n_out, nj, s, j > 0);
             if (rc != RMI_OK) return rc;
         }
         return RMI_OK;

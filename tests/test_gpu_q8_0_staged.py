@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("ncols,res", [(1, False), (1, True), (2, False), (2, True)])
 @pytest.mark.parametrize("n_in,n_out", [(2048, 5121), (4096, 2561), (4096, 4096), (4352, 4099), (12288, 1001),
-                                        (28928, 402), (29184, 401), (2048, 4882), (2048, 4883)])
+                                        (28928, 402), (29184, 401), (2048, 4882), (2048, 4883), (2048, 5371), (2048, 5441),
+                                        (2304, 4341)])
 def test_staged_is_the_general_kernel(ncols, res, n_in, n_out):
     import oracle
     import rapier_amd as rmi
@@ -41,3 +42,9 @@ def test_staged_is_the_general_kernel(ncols, res, n_in, n_out):
     assert T.equal(y[0], y[1])
     if res:
         assert T.equal(part[0], part[1])
+
+
+@pytest.mark.parametrize("ncols", [5, 6])
+@pytest.mark.parametrize("n_in,n_out", [(16384, 1279), (16384, 1281)])   # both sides of the line for a last pass
+def test_last_pass_of_more_columns(ncols, n_in, n_out):
+    test_staged_is_the_general_kernel(ncols, True, n_in, n_out)
