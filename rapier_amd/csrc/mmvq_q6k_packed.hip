@@ -903,15 +903,19 @@ __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
 // lane (row i, group g, column jj) adds its 16 half-blocks in the xor butterfly's tree (bitwise hb_sum), then owns one
 // output: ~60 instructions per quad where the 16 in-register butterflies take ~300.  Needs 4 KB x NCW of LDS per wave:
 // after the stage, or with two K halves the stage itself once every wave is past its last chunk.
-template <int NCG, bool RES, int D, int CS = 1, int KP = 1, int NCHK = 0, bool LE = false>
+// PART: a part-full pass of ncols < 4 NCG columns.  Full passes compile without its clamps (they cost them 0.2 us: 6144 x
+// 512 with 8 columns 8.5 -> 8.9).
+template <int NCG, bool RES, bool PART, int D, int CS = 1, int KP = 1, int NCHK = 0, bool LE = false>
 __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t* __restrict__ wp,
                                                                    const uint8_t* __restrict__ x, float* y,
                                                                    const float* res, float* partials, int n_in,
-                                                                   int n_out, int ncols) {
+                                                                   int n_out, int ncols_part) {
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     static_assert(CS == 1 || CS == 2, "column split: one or two waves per quad");
     static_assert(KP == 1 || (KP == 2 && CS == 2 && NCHK % 2 == 0 && NCHK > 0), "two K halves: a wave pair per quad");
     static_assert(!LE || NCG / CS <= 4, "LDS row sums: at most 64 outputs per wave");
+    const int ncols = PART ? ncols_part : 4 * NCG;
+    auto src_col = [&](int col) { return PART ? min(col, ncols - 1) : col; };
     constexpr int NCW = NCG / CS;            // column groups of this wave
     constexpr int PG = NCW >= 2 ? 2 : 1;     // column groups per MFMA batch
     extern __shared__ uint4 smem[];   // the stage may take all 160 KB of the CU's LDS: no static LDS
@@ -938,7 +942,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
     for (int m = 0; m < kStageRegs; ++m) {
         const int J = min(t + 64 * kWideWaves * m, nb_stage - 1);
         const int col = J / nbs_stage, jb = J - col * nbs_stage;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + jb) * kQ8_1Bytes);
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(src_col(col) * nbt + jb) * kQ8_1Bytes);
 #pragma unroll
         for (int i = 0; i < 9; ++i) sv[m][i] = p[i];
     }
@@ -972,7 +976,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
     }
     for (int J = t + 64 * kWideWaves * kStageRegs; J < nb_stage; J += 64 * kWideWaves) {
         const int col = J / nbs_stage, jb = J - col * nbs_stage;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + jb) * kQ8_1Bytes);
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(src_col(col) * nbt + jb) * kQ8_1Bytes);
         uint32_t wv[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) wv[i] = p[i];
@@ -988,7 +992,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
             const int J = min(t + 64 * kWideWaves * m, nb - 1);
             const int col = J / nbs, jb = J - col * nbs;
             const uint32_t* p =
-                reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(min(col, ncols - 1) * nbt + nbs + jb) * kQ8_1Bytes);
+                reinterpret_cast<const uint32_t*>(x + static_cast<size_t>(src_col(col) * nbt + nbs + jb) * kQ8_1Bytes);
 #pragma unroll
             for (int i = 0; i < 9; ++i) pb[m][i] = p[i];
         }
@@ -1113,7 +1117,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
                 // lane o: row io = o / R, group go = (o / 4) % NCW, column jo = o % 4 (lanes past 16 NCW idle)
                 const int oo = lane < 4 * R ? lane : 0;
                 const int io = oo / R, go = (oo >> 2) % NCW, jo = oo & 3;
-                const bool live = lane < 4 * R && 4 * (NCW * half + go) + jo < ncols;
+                const bool live = lane < 4 * R && (!PART || 4 * (NCW * half + go) + jo < ncols);
                 float hv[16];
 #pragma unroll
                 for (int h = 0; h < 16; ++h) hv[h] = lescr[(4 * h + jo) * R + io * NCW + go];
@@ -1157,12 +1161,12 @@ __global__ __launch_bounds__(64 * kWideWaves) void q6k_packed_mfma(const uint8_t
                         tot[i][g] = 0.0f;
                         const int row = kQuad * q + i;
                         if constexpr (RES) {
-                            if (row < n_out && col < ncols) v[i] += res[static_cast<size_t>(col) * n_out + row];
+                            if (row < n_out && (!PART || col < ncols)) v[i] += res[static_cast<size_t>(col) * n_out + row];
                         }
-                        if (hb == 0 && row < n_out && col < ncols) y[static_cast<size_t>(col) * n_out + row] = v[i];
+                        if (hb == 0 && row < n_out && (!PART || col < ncols)) y[static_cast<size_t>(col) * n_out + row] = v[i];
                     }
                     if constexpr (RES) {
-                        if (hb == 0 && col < ncols) {   // squares of the quad's rows in row order
+                        if (hb == 0 && (!PART || col < ncols)) {   // squares of the quad's rows in row order
                             const int row0 = kQuad * q;
                             float p = __builtin_fmaf(v[0], v[0], 0.0f);
                             if (row0 + 1 < n_out) p = __builtin_fmaf(v[1], v[1], p);
@@ -1339,15 +1343,15 @@ int wide_grid(int nq, int units_per_wg) {
     return (units + units_per_wg - 1) / units_per_wg;
 }
 
-template <int NCOLS, bool RES>
+template <int NCOLS, bool RES, bool PART>
 int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const float* res, float* partials, int n_in,
                        int n_out, int ncols, hipStream_t s) {
     constexpr int D = 3;
     constexpr int NCG = NCOLS / 4;
-    auto kern = q6k_packed_mfma<NCG, RES, D>;
-    auto kern2 = q6k_packed_mfma<NCG, RES, D, 2>;
-    auto kernl = q6k_packed_mfma<NCG, RES, D, 1, 1, 0, true>;
-    auto kern2l = q6k_packed_mfma<NCG, RES, D, 2, 1, 0, true>;
+    auto kern = q6k_packed_mfma<NCG, RES, PART, D>;
+    auto kern2 = q6k_packed_mfma<NCG, RES, PART, D, 2>;
+    auto kernl = q6k_packed_mfma<NCG, RES, PART, D, 1, 1, 0, true>;
+    auto kern2l = q6k_packed_mfma<NCG, RES, PART, D, 2, 1, 0, true>;
     auto lds_attr = [](auto k) {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    kWideStageBytes) == hipSuccess;
@@ -1363,8 +1367,8 @@ int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const floa
         if constexpr (NCOLS == 16) {
             // two K halves, a wave pair per quad (the second half's blocks take 54 registers: one tile fewer in flight)
             // (the LDS row sums reuse the stage after the last chunk)
-            auto kh4 = q6k_packed_mfma<4, RES, 2, 2, 2, 4, true>;
-            auto kh6 = q6k_packed_mfma<4, RES, 2, 2, 2, 6, true>;
+            auto kh4 = q6k_packed_mfma<4, RES, PART, 2, 2, 2, 4, true>;
+            auto kh6 = q6k_packed_mfma<4, RES, PART, 2, 2, 2, 6, true>;
             static const bool attr_h = lds_attr(kh4) && lds_attr(kh6);
             if (!attr_h) return fail(RMI_ERR_LAUNCH, "native_q6_k_mmvq_packed: wide LDS stage not available");
             if (wide_halves(n_in, n_out)) {
@@ -1420,8 +1424,9 @@ int run_packed(const void* wpv, const void* xv, float* y, const float* res, floa
         const float* rj = RES ? res + static_cast<size_t>(j) * n_out : nullptr;
         float* pj = RES ? partials + j * pcol : nullptr;
         if (wide) {
-            const int rc = wide == 8 ? launch_packed_wide<8, RES>(wp, xj, yj, rj, pj, n_in, n_out, nj, s)
-                                     : launch_packed_wide<16, RES>(wp, xj, yj, rj, pj, n_in, n_out, nj, s);
+            const auto pass = wide == 8 ? (nj == 8 ? launch_packed_wide<8, RES, false> : launch_packed_wide<8, RES, true>)
+                                        : (nj == 16 ? launch_packed_wide<16, RES, false> : launch_packed_wide<16, RES, true>);
+            const int rc = pass(wp, xj, yj, rj, pj, n_in, n_out, nj, s);
             if (rc) return rc;
         } else {
             switch (nj) {
