@@ -339,12 +339,9 @@ int q6k_packed_gemm(const void* w_packed, const void* x_q8_1, float* y, const fl
                        static_cast<const uint8_t*>(x_q8_1), xc, xd, nbt, ncols, tpad);
     RMI_TRY(launch_status("q6_k_gemm_packed"));
     constexpr int lds = 4 * static_cast<int>(sizeof(Step));
-    static const bool attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(q6k_ingest_gemm<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            lds) == hipSuccess &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(q6k_ingest_gemm<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            lds) == hipSuccess;
-    if (!attr) return fail(RMI_ERR_LAUNCH, "q6_k_gemm_packed: LDS not available");
+    static OncePerDevice attr;
+    if (!attr([] { return lds_limit(q6k_ingest_gemm<true>, lds) && lds_limit(q6k_ingest_gemm<false>, lds); }))
+        return fail(RMI_ERR_LAUNCH, "q6_k_gemm_packed: LDS not available");
     const int ct = tpad / kTileCols, rt = (n_out + kTileRows - 1) / kTileRows;
     const auto* wp = static_cast<const uint8_t*>(w_packed);
     if (res)

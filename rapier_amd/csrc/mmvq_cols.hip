@@ -411,9 +411,8 @@ int launch(const uint8_t* w, const uint8_t* x, float* y, const float* res, float
     constexpr int lds = NS * kSlabBlocks * table_row(TYPE) * 4 + std::max(tiles_bytes, 16 * kSlabCol * 4);
     static_assert(lds <= kMaxLds, "LDS");
     auto k = cols_gemv_kernel<TYPE, NLU, NS, RES>;
-    static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 kMaxLds) == hipSuccess;
-    if (!attr) return fail(RMI_ERR_LAUNCH, "native MMVQ: LDS not available");
+    static OncePerDevice attr;
+    if (!attr([&] { return lds_limit(k, kMaxLds); })) return fail(RMI_ERR_LAUNCH, "native MMVQ: LDS not available");
     const int tiles = (n_out + 15) / 16, per = (tiles + kMaxWgs - 1) / kMaxWgs;
     hipLaunchKernelGGL(k, dim3((tiles + per - 1) / per), dim3(64 * kWaves), lds, s, w, x, y, res, partials, n_in, n_out, ncols,
                        tiles);

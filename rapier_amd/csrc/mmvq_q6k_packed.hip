@@ -1352,12 +1352,12 @@ int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const floa
     auto kern2 = q6k_packed_mfma<NCG, RES, PART, D, 2>;
     auto kernl = q6k_packed_mfma<NCG, RES, PART, D, 1, 1, 0, true>;
     auto kern2l = q6k_packed_mfma<NCG, RES, PART, D, 2, 1, 0, true>;
-    auto lds_attr = [](auto k) {
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   kWideStageBytes) == hipSuccess;
-    };
-    static const bool attr = lds_attr(kern) && lds_attr(kern2) && lds_attr(kernl) && lds_attr(kern2l);
-    if (!attr) return fail(RMI_ERR_LAUNCH, "native_q6_k_mmvq_packed: wide LDS stage not available");
+    static OncePerDevice attr;
+    if (!attr([&] {
+            return lds_limit(kern, kWideStageBytes) && lds_limit(kern2, kWideStageBytes) && lds_limit(kernl, kWideStageBytes) &&
+                   lds_limit(kern2l, kWideStageBytes);
+        }))
+        return fail(RMI_ERR_LAUNCH, "native_q6_k_mmvq_packed: wide LDS stage not available");
     // the LDS row sums (LE) where their scratch, 4 KB per column group of a wave, fits after the stage
     static const bool le_on = env_int("RMI_WIDE_LE", 1) != 0;
     auto le_bytes = [](int ncw) { return static_cast<size_t>(kWideWaves) * 64 * 4 * ncw * sizeof(float); };
@@ -1369,8 +1369,9 @@ int launch_packed_wide(const uint8_t* wp, const uint8_t* x, float* y, const floa
             // (the LDS row sums reuse the stage after the last chunk)
             auto kh4 = q6k_packed_mfma<4, RES, PART, 2, 2, 2, 4, true>;
             auto kh6 = q6k_packed_mfma<4, RES, PART, 2, 2, 2, 6, true>;
-            static const bool attr_h = lds_attr(kh4) && lds_attr(kh6);
-            if (!attr_h) return fail(RMI_ERR_LAUNCH, "native_q6_k_mmvq_packed: wide LDS stage not available");
+            static OncePerDevice attr_h;
+            if (!attr_h([&] { return lds_limit(kh4, kWideStageBytes) && lds_limit(kh6, kWideStageBytes); }))
+                return fail(RMI_ERR_LAUNCH, "native_q6_k_mmvq_packed: wide LDS stage not available");
             if (wide_halves(n_in, n_out)) {
                 const dim3 grid((nq + kWideWaves / 2 - 1) / (kWideWaves / 2)), block(64 * kWideWaves);
                 if (lds / 2 < le_bytes(2)) return fail(RMI_ERR_SHAPE, "native_q6_k_mmvq_packed: half stage too small");

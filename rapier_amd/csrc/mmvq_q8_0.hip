@@ -189,25 +189,25 @@ __global__ __launch_bounds__(64 * W) void q8_0_gemv_staged(const uint4* __restri
 }
 
 template <int NCOLS, bool RES, int W>
-void launch_staged(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials, int n_in, int n_out,
-                   hipStream_t s) {
+int launch_staged(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials, int n_in, int n_out,
+                  hipStream_t s) {
     // the columns' LDS limit and the row areas together exceed the default 64 KB
-    static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(q8_0_gemv_staged<NCOLS, RES, W>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 W * kPieces * 16 + kStagedMax) == hipSuccess;
-    (void)attr;
+    static OncePerDevice attr;
+    if (!attr([] { return lds_limit(q8_0_gemv_staged<NCOLS, RES, W>, W * kPieces * 16 + kStagedMax); }))
+        return fail(RMI_ERR_LAUNCH, "native_q8_0_mmvq: LDS not available");
     const size_t lds = static_cast<size_t>(W) * kPieces * 16 + static_cast<size_t>(NCOLS) * (n_in / 32) * kQ8_1Bytes;
     hipLaunchKernelGGL((q8_0_gemv_staged<NCOLS, RES, W>), dim3((n_out + W - 1) / W), dim3(64 * W), lds, s,
                        reinterpret_cast<const uint4*>(w), reinterpret_cast<const uint4*>(x), y, res, partials, n_in, n_out);
+    return launch_status("native_q8_0_mmvq");
 }
 
 // W: as many rows per workgroup as leave a workgroup for each of the 256 CUs
 template <int NCOLS, bool RES>
-void launch_staged(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials, int n_in, int n_out,
-                   hipStream_t s) {
-    if (n_out >= 16 * 256) launch_staged<NCOLS, RES, 16>(w, x, y, res, partials, n_in, n_out, s);
-    else if (n_out >= 8 * 256) launch_staged<NCOLS, RES, 8>(w, x, y, res, partials, n_in, n_out, s);
-    else launch_staged<NCOLS, RES, 4>(w, x, y, res, partials, n_in, n_out, s);
+int launch_staged(const uint8_t* w, const uint8_t* x, float* y, const float* res, float* partials, int n_in, int n_out,
+                  hipStream_t s) {
+    if (n_out >= 16 * 256) return launch_staged<NCOLS, RES, 16>(w, x, y, res, partials, n_in, n_out, s);
+    if (n_out >= 8 * 256) return launch_staged<NCOLS, RES, 8>(w, x, y, res, partials, n_in, n_out, s);
+    return launch_staged<NCOLS, RES, 4>(w, x, y, res, partials, n_in, n_out, s);
 }
 
 // Matrices the staged kernel takes: whole aligned pieces, the columns within their LDS, rows of half a step or more, and
@@ -233,11 +233,9 @@ int launch(const void* wv, const void* xv, float* y, const float* res, float* pa
     if (ncols > 2)
         if (const int rc = cols_gemv(8, 64, w, x, y, res, partials, n_in, n_out, ncols, s); rc >= 0)
             return rc;
-    if (ncols <= 2 && staged(w, x, n_in, n_out, ncols, behind)) {
-        if (ncols == 1) launch_staged<1, RES>(w, x, y, res, partials, n_in, n_out, s);
-        else launch_staged<2, RES>(w, x, y, res, partials, n_in, n_out, s);
-        return launch_status("native_q8_0_mmvq");
-    }
+    if (ncols <= 2 && staged(w, x, n_in, n_out, ncols, behind))
+        return ncols == 1 ? launch_staged<1, RES>(w, x, y, res, partials, n_in, n_out, s)
+                          : launch_staged<2, RES>(w, x, y, res, partials, n_in, n_out, s);
     if (ncols > 4) {
         const size_t xcol = static_cast<size_t>(n_in / 32) * kQ8_1Bytes;
         const size_t pcol = static_cast<size_t>((n_out + 3) / 4);

@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 
@@ -32,6 +33,31 @@ int launch_status(const char* what);   // hipGetLastError after a launch -> RMI_
 
 inline bool aligned4(const void* p) { return p && (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 inline bool aligned16(const void* p) { return p && (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Something to do once per device, e.g. raising kernels' dynamic LDS limits: the attribute belongs to the current device's copy
+// of a kernel, so a process that calls on a second device needs it there too.  Threads may race to the same call.
+class OncePerDevice {
+    std::atomic<uint64_t> done_[4] = {};
+
+public:
+    template <typename F>
+    bool operator()(F&& what) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 256) return what();
+        std::atomic<uint64_t>& w = done_[dev >> 6];
+        const uint64_t bit = uint64_t(1) << (dev & 63);
+        if (w.load(std::memory_order_acquire) & bit) return true;
+        if (!what()) return false;
+        w.fetch_or(bit, std::memory_order_release);
+        return true;
+    }
+};
+
+template <typename K>
+bool lds_limit(K* kernel, int bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) ==
+           hipSuccess;
+}
 
 // ---- device helpers ----
 __device__ __forceinline__ float half_bits_to_float(uint32_t bits) {
