@@ -88,3 +88,23 @@ def test_kernel_argument_validation(rmi):
                   ctypes.c_float(0.0625), FAKE)
     with pytest.raises(ValueError, match="bad shape"):
         rmi._call("rmi_argmax", FAKE, 0, 1, 0, FAKE, FAKE, FAKE)
+
+
+def test_packed_gemm_argument_validation(rmi):
+    off = ctypes.c_void_p((1 << 20) + 4)   # not 16-byte aligned
+
+    def call(w=FAKE, x=FAKE, y=FAKE, res=FAKE, part=FAKE, n_in=2048, n_out=8, ncols=17, ws=FAKE, stream=FAKE):
+        rmi._call("rmi_q6_k_gemm_packed", w, x, y, res, part, n_in, n_out, ncols, ws, stream)
+
+    for bad in ({"n_in": 256}, {"n_in": 0}, {"n_out": 0}, {"ncols": 0}, {"ncols": 4097}):
+        with pytest.raises(ValueError, match="n_in must be a positive multiple of 2048"):
+            call(**bad)
+    for bad in ({"w": None}, {"x": None}, {"y": None}, {"ws": None}, {"part": None}, {"w": off}, {"y": off}, {"ws": off},
+                {"res": off}):
+        with pytest.raises(ValueError, match="null or misaligned"):
+            call(**bad)
+    with pytest.raises(ValueError, match="stream"):
+        call(stream=None)
+    for bad in ((100, 17), (2048, 0)):
+        with pytest.raises(ValueError):
+            rmi.q6_k_gemm_workspace_bytes(*bad)

@@ -116,8 +116,8 @@ def test_qwen35_9b_mtp_stream_bit_identical_at_64k(eng_mod, engine_64k):
 
 
 def test_qwen35_9b_mtp_after_ingest_past_32k(eng_mod, engine_64k):
-    """a random prompt of 33,000 tokens ingested in 16-token chunks (every GEMV, GDN step and attention chunk of the
-    batched path, the context past 32K), then MTP at forced acceptance 0 / 0.5 / 1.0 equals greedy"""
+    """a random prompt of 33,000 tokens ingested in wide chunks (the GEMM, GDN scan and attention chunks of the wide path,
+    the context past 32K), then MTP at forced acceptance 0 / 0.5 / 1.0 equals greedy"""
     E, eng = eng_mod, engine_64k
     prompt = [int(t) for t in np.random.default_rng(17).integers(0, 248320, size=33000)]
     first = eng.prefill(prompt, batch=16)
