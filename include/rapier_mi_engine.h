@@ -71,6 +71,8 @@ typedef struct rmi_gen_stats {
 } rmi_gen_stats;
 
 rmi_model_config rmi_qwen35_9b_config(void);
+/* Beside weights, caches and state an engine whose matrices are all packed Q6_K holds the buffers of prompt chunks of
+ * min(1024, max_ctx) tokens: 0.39 GB for the 9B model at max_ctx 4096 (8.4 GB in all), 0.44 GB at 66000 (10.7 GB). */
 int rmi_engine_create(const rmi_model_config* cfg, uint64_t seed, int max_ctx, void* stream, rmi_engine** out);
 int rmi_engine_destroy(rmi_engine* e);
 int rmi_engine_info(const rmi_engine* e, rmi_engine_info_t* info);

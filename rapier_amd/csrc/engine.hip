@@ -37,11 +37,12 @@ namespace {
 constexpr int kS = 128;          // GDN state size
 constexpr int kRingCap = 1 << 16;
 constexpr int kChunk = kMaxCols;  // ingest chunk: prompt tokens per weight pass
-// Wide ingest chunks: up to kWideCols tokens per pass over the weights, while at least kWideMin are left (below that
-// the GEMM's 128-column tile costs more than the 16-column passes).  1999 tokens of the 9B model: 456 -> 141 ms.
+// Wide ingest chunks: up to kWideCols tokens per pass over the weights, while at least kWideMin are left.  9B model, wide /
+// in 16-token chunks: 64 tokens 15.1 / 16.0 ms, 80 15.4 / 20.0, 128 16.1 / 31.2, 129 (a second column tile) 19.8 / 33.0, 1999
+// 131 / 487; small test model 64 tokens 1.22 / 1.52 ms; 64 tokens behind 33,000 positions 17.1 / 20.1.
 constexpr int kWideCols = 1024;
 constexpr int kWideMin = 64;
-constexpr int kWideAttnTok = 128;   // tokens per attention launch of a wide chunk (its split-K records: 64 MiB at 2K)
+constexpr int kWideAttnTok = 128;   // tokens per attention launch of a wide chunk (9B split-K records: 36 MB at 2K, 136 MB at 64K)
 constexpr int kAttnSlots = 64;    // query vectors per KV head one rmi_gqa_flash_decode launch takes
 
 int hip_check(hipError_t e, const char* what) {

@@ -439,8 +439,8 @@ __global__ __launch_bounds__(S * RG) void gdn_step_kernel(StepArgs a) {
 // 128 rows in two waves (lane: column 32 part + 16 w + l % 16, row group l / 16), so 128 CUs carry the state instead
 // of 32 and each SIMD one wave instead of two.  Every per-lane operation, and every reduction order, is that of
 // gdn_step_kernel (the column sums over row groups, the conv's 64-lane L2 partials, the output norm's sum of the eight
-// 16-column wave sums in wave order), so the results are bitwise those of the one-workgroup kernel, which the ingest
-// chunks run.  The part's 32 columns are one Q8_1 block per token.
+// 16-column wave sums in wave order), so the results are bitwise those of the one-workgroup kernel, which chunks of 3..5
+// tokens run.  The part's 32 columns are one Q8_1 block per token.
 // Each part recomputes the head's q and k conv (all 128 channels: the step reads all of them); part 0 writes their
 // history once the exchange shows that every other part has used the history it loaded.  The output norm needs the head's eight wave sums: each part publishes its two per token as {bits, epoch}
 // 8-byte words (agent scope: value and tag land together) and reads the other parts' words.  The epoch is the number
@@ -1156,7 +1156,8 @@ extern "C" int rmi_fused_gdn_step_norm_silu_q8(float* state, const float* q, con
 
 // ---- engine surface: qkv|z and beta|alpha GEMV outputs, 1..16 tokens, selector-based rollback buffers --------------
 // ntok = 2 is the verify pair (after-token-0 state and history to the non-live buffers); 1 and 3..16 update the live
-// buffers in place (3..16: an ingest chunk, the row-batched step of src/qwythos_ingest.cu).  Per token t: qkvz + t * qkvz_stride holds [q h_k*128 | k h_k*128 | v h_v*128 | z h_v*128]; ab + t * ab_stride holds
+// buffers in place (3..16: an ingest chunk, the row-batched step of src/qwythos_ingest.cu).  Per token t: qkvz + t *
+// qkvz_stride holds [q h_k*128 | k h_k*128 | v h_v*128 | z h_v*128]; ab + t * ab_stride holds
 // [beta h_v | alpha h_v] (both read only).  History per value head, [h_v][3 * 128][3].  Output y + t * y_stride, q8
 // + t * q8_stride.
 namespace {

@@ -17,11 +17,13 @@
 //    once per 128 columns.  A step is one half-block of the tile: 64 rows' codes as digits (16 KB) and 128 columns'
 //    codes (16 KB) per group, double-buffered in LDS; the next step's loads (the columns straight into LDS) fly during
 //    the MFMAs.
-//  * Bound: the vector unit.  Per output and Q8_1 block a shift-add, a convert and an fma (192 cycles per 32x32x32 cell
-//    and SIMD against 64 of MFMA), plus ~50 for unpacking the weights at 128 columns.  24576 x 4096 at 1024 columns:
+//  * Bound: the vector unit, 71% busy (two waves per SIMD; they wait 35% of their cycles). Per 32x32x32 cell 85 vector
+//    instructions (340 cycles of a SIMD) against 64 cycles of MFMA: a shift-add, a convert and an fma per output and Q8_1
+//    block are 48 of them, the rest unpacks weights (once per 128 columns), folds and moves.  24576 x 4096 at 1024 columns:
 //    642 us (0.32 Pop/s) where 64 passes of the 16-column kernel take 1690 us; 4096 x 12288: 300 us (64 x 22.4).
-//  * From 64 columns: a tile costs the same whatever its columns (24576 x 4096: 107 us at 1..128), the 16-column kernel
-//    26 us per pass.
+//  * A tile costs the same whatever its columns (24576 x 4096: 107 us at 1..128, four 16-column passes 104), and matrices
+//    of 4096 rows fill 64 CUs per 128 columns.  Over all matrices of the 9B model it wins from 64 columns (15.1 ms for a
+//    64-token prompt, 16.0 in 16-column passes; 128 tokens 16.1 / 31.2).
 #include "rmi_common.h"
 #include "ingest.h"
 

@@ -1327,6 +1327,7 @@ int cols_per_pass(int n_in) {
 // takes.  A part-full pass stages its last column in the missing ones' place and stores nothing for them: 4096 x 12352
 // with 5 columns 23.1 -> 15.5 us (4 + 1 before), 9 columns 24.0 -> 20.0 (8 + 1), 15 columns 40.7 -> 20.1 (8 + 4 + 3);
 // 12288 x 4096 with 4 columns 22.0 -> 17.4 (3 + 1).  One narrow pass stays the faster one (3 / 4 columns 13.4 / 14.6).
+// Over 31 shapes from 2048 x 512 and 4096 x 256 to 16384 x 4096 no count of 3..16 columns got slower (geometric mean 0.80).
 int wide_cols(int n_in, int n_out, int remaining) {
     if (remaining > 8 && (wide_stage_bytes(n_in, 16) <= kWideStageBytes || wide_halves(n_in, n_out))) return 16;
     if (remaining > cols_per_pass(n_in) && wide_stage_bytes(n_in, 8) <= kWideStageBytes) return 8;
