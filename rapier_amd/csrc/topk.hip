@@ -16,8 +16,8 @@
 // of both, and a bitonic half-cleaner network (lane strides 32 .. 1) sorts them; B is kept ascending, so no lane
 // reversal is needed.
 // All are bound by their chains of exchanges.  Both launches, networks / popping: 248320 logits k = 1 13.6 / 10.1 us, k = 16
-// 13.6 / 13.2, k = 24 13.6 / 14.9, k = 40 13.7 / 18.3; 1000 logits k = 1 8.6 / 4.8, k = 16 8.5 / 8.0, k = 20 8.6 / 8.8.  Merging the lists pair by
-// pair through LDS took 12.4 us at 248320 logits (7.3 here).
+// 13.6 / 13.2, k = 24 13.6 / 14.9, k = 40 13.7 / 18.3; 1000 logits k = 1 8.6 / 4.8, k = 16 8.5 / 8.0, k = 20 8.6 / 8.8.
+// Merging the lists pair by pair through LDS took 12.4 us at 248320 logits (6.5 to 7.3 here).
 #include "rmi_common.h"
 
 #include <type_traits>
